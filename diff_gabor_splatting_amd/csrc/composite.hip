@@ -28,10 +28,13 @@
 //    pre-activations folded to zc + U u + V v;
 //  * reciprocals (v_rcp) replace the IEEE divisions and exp2 replaces expf
 //    (both within two float32 ulps);
-//  * in the backward, each wave sums its 64 pixels' gradients with one
-//    reduce-scatter (wave.hpp), adds them to a per-batch LDS accumulator with
-//    one ds_add per wave, and after the batch the workgroup flushes nonzero
-//    totals with one global atomic per (tile, record, parameter).
+//  * in the neural backward (and full-list walks), each wave sums its 64
+//    pixels' gradients with one reduce-scatter (wave.hpp), adds them to a
+//    per-batch LDS accumulator with one ds_add per wave, and after the batch
+//    the workgroup flushes nonzero totals with one global atomic per (tile,
+//    record, parameter);
+//  * the classic replay backward puts 16 records x 4 pixels on a wave's lanes,
+//    so that a record's sums over its pixels stay in registers (by_record).
 #include <climits>
 #include <cmath>
 #include <mutex>
@@ -169,15 +172,14 @@ __device__ __forceinline__ float fract(float t) { return __builtin_amdgcn_fractf
 // SUM_c), the backward's rows hold SUM_c and HALF_W for the flush and the
 // product at SUMW.
 // THR (reject_threshold of the opacity) is written only for the full-list
-// backward, the one reader of it (sample_surface with Reject); the replay
-// backward keeps the record's list position in that slot instead (POS), so
-// that it arrives with the row's other constants rather than in a separate
+// backward, the one reader of it (sample_surface with Reject); the neural
+// replay backward keeps the record's list position in that slot instead (POS),
+// so that it arrives with the row's other constants rather than in a separate
 // dependent load.
 struct ClassicRow {
   static constexpr int OP = 14, THR = 15;
   static constexpr int A = 16, B = 20, C = 24, HW = 28;  // 4 each
   static constexpr int HALF_W = 32, SUM = 33, DIFF = 36;  // 1, 3, 3
-  static constexpr int POS = THR;  // replay backward: the record's list position (int bits)
   static constexpr int AP = 40, BP = 44;  // -2 pi HW_f A_f, -2 pi HW_f B_f (backward)
   static constexpr int SUMW = 48;         // HALF_W SUM_c (backward)
   static constexpr int STRIDE = 52;
@@ -747,8 +749,6 @@ __device__ __forceinline__ uint64_t load_batch(float* rows, float* raw, float* r
       for (int i = 0; i < 3; ++i) r[R::B2 + i] = a[54 + i];
     } else {
       using R = ClassicRow;
-      if constexpr (Which == kReplayMask)
-        r[R::POS] = __int_as_float(entries[t] & kReplayPositionMask);
       r[R::OP] = opacity;
       if constexpr (kRowThreshold) r[R::THR] = reject_threshold(opacity);
       float half_w = 0.f;
@@ -1717,13 +1717,12 @@ __device__ __forceinline__ float classic_appearance_gradient(const float* sums, 
 // range start, replay_counts[tile] entries) instead of its point list up to
 // tile_last[tile], compositing each record only in the quadrants that took
 // it; tile_last is then unused.
-// Workgroups per CU: the classic replay walk runs six (25.1 KB of LDS each;
-// the compiler holds it to 80 VGPRs and spills only outside the record loop,
-// which stays free of scratch), the others four, or two for the neural
-// full-list walk.
+// Used for the neural renderer and for full-list walks; the classic replay
+// walk is by_record::renderBackward. Workgroups per CU: four, or two for the
+// neural full-list walk.
 template <bool Neural, bool Replay>
 constexpr int backward_occupancy() {
-  return Neural ? (Replay ? 4 : 2) : (Replay ? 6 : 4);
+  return Neural && !Replay ? 2 : 4;
 }
 
 template <bool Neural, bool Replay>
@@ -1739,6 +1738,7 @@ __global__ __launch_bounds__(kTilePixels, (backward_occupancy<Neural, Replay>())
     float* __restrict__ grad_geometry, const AppearanceGradient grad_appearance,
     float* __restrict__ grad_opacities, float* __restrict__ grad_backgrounds,
     const int2* __restrict__ segments, Segments seg) {
+  static_assert(Neural || !Replay, "the classic replay walk is by_record::renderBackward");
   using L = Layout<Neural>;
   constexpr int NP = L::NP;
   constexpr int NG = L::NG;
@@ -1929,7 +1929,7 @@ __global__ __launch_bounds__(kTilePixels, (backward_occupancy<Neural, Replay>())
       // List position of row j, counted from 1.
       int position = start - j;
       if constexpr (Replay)
-        position = __float_as_int(r[Neural ? NeuralRow::POS : ClassicRow::POS]) + 1;
+        position = __float_as_int(r[NeuralRow::POS]) + 1;
       // A replayed record was taken in the forward by a pixel of this wave's
       // quadrant, so some lane accepts it again and the wave-wide tests are
       // skipped (were none to accept, the stand-ins would make the adjoint
@@ -2168,6 +2168,689 @@ __global__ __launch_bounds__(kTilePixels, (backward_occupancy<Neural, Replay>())
   stamp_tile(gs_diagnostics.backward_span, tile, diag_begin);
 #endif
 }
+
+// The classic replay backward: the lanes of a wave are 16 records x 4 pixels.
+//
+// One wave takes one 8x8 quadrant of a tile and walks the quadrant's replay
+// entries (the records that some pixel of it took) from the last to the
+// first, 16 records at a time. Lane l holds record l & 15 of the chunk in
+// registers, and the wave steps through the quadrant's pixels four at a time,
+// lane l evaluating pixel 4 g + (l >> 4) in step g:
+//  * a record's gradient is a sum over pixels, and a lane keeps its record
+//    for all 16 steps, so every summand is one multiply-add into a register;
+//    what remains of the reduction is one sum over four lanes per chunk.
+//    With a pixel per lane, the 64-lane reduction of every record took 79 of
+//    its 253 instructions, and every lane read the record's row (13 16-byte
+//    LDS reads per record and wave);
+//  * what couples a pixel's records is its transmittance and the running sum
+//    of w dL/dw behind a record. Over the chunk's 16 lanes they are an
+//    inclusive product scan of 1 / (1 - alpha) and an exclusive sum scan
+//    (four DPP steps each within the 16-lane row); a pixel's state between
+//    chunks stays in LDS;
+//  * per step a lane reads its pixel's 16 constants (four 16-byte LDS reads,
+//    one address per 16-lane row).
+// The waves of a workgroup share nothing but the tile, so there is no barrier
+// after the prologue and no batch: each wave ends when its own list does.
+//
+// It is bound by VALU issue: about 170 instructions per step of 64 samples and
+// 300 per chunk around the steps, against 253 per record and wave with a pixel
+// per lane. Measured, kernel alone: 1M surfels at 1920x1080, all maps, 1.167 ->
+// 0.986 ms; 100k at 1024x768, rgb, alpha and depth, 0.448 -> 0.388 ms; 32 views
+// at 512x512 4.74 -> 4.01 ms. Three waves per SIMD without spills are 2% faster
+// than four with 14 spilled registers. The neural adjoint has 57 sums and 55
+// record constants, which leave two waves per SIMD, and stays with a pixel per
+// lane (0.684 ms against 0.714 on 100k surfels at 800x800). An f32 MFMA per four
+// pixels in place of the products with per-pixel values (20 multiply-adds for 6
+// MFMAs) is slower (1.23 ms): each takes its 32 cycles of the SIMD.
+namespace by_record {
+
+constexpr int kChunk = 16;              // records per chunk: one DPP row
+constexpr int kGroups = 64 / 4;         // pixel steps per chunk
+constexpr int kQueue = 128;             // ring of filtered replay entries per wave
+
+// A pixel's constants in LDS: position, last contributor (int bits), the
+// term of dL/dalpha that all records share, map gradients (rgb, depth,
+// normals) and the depth and distortion factors (see depth_terms).
+struct ReplayPixel {
+  static constexpr int RGB = 0, NORMAL = 3;
+  static constexpr int X = 6, Y = 7, LAST = 8, FINAL = 9, DEPTH = 10;
+  static constexpr int A8 = 11, C8 = 12, D8 = 13, E8 = 14, F8 = 15;
+  static constexpr int FLOATS = 16;
+};
+
+// Which maps have gradients: the step leaves out the terms of the others
+// (normals and distortion: 14 of 168 instructions; depth: 8 more).
+constexpr int kColour = 0;       // rgb, alpha
+constexpr int kColourDepth = 1;  // and depth
+constexpr int kAllMaps = 2;      // and normals or distortion
+
+// The sums that a lane accumulates over its record's pixels.
+//  G, X, Y: sum gp, sum dx gp, sum dy gp of the adjoint gp of p = k x l, with
+//    (dx, dy) the record's centre minus the pixel: k = x T2 - T0 and
+//    l = y T2 - T1 are affine in (dx, dy), so these nine sums give the
+//    gradients of the three rows of T (record_gradients).
+//  XY: the screen filter's centre; OPACITY.
+//  APPEARANCE: sum w g_c, sum w S g_c, and per frequency sum cos g, sum sin g
+//    dot, sum sin g (see record_gradients).
+//  TILT: sum gz s_u, gz s_v, gz (T's last row through the depth); NORMAL.
+template <int Maps>
+struct Sums {
+  static constexpr int G = 0, X = 3, Y = 6, XY = 9, OPACITY = 11, APPEARANCE = 12;
+  static constexpr int TILT = 30, NORMAL = 33;
+  static constexpr int COUNT = Maps == kAllMaps ? 36 : Maps == kColourDepth ? 33 : 30;
+};
+
+// Inclusive scans over the 16 lanes of a DPP row: lanes whose source lies
+// before the row keep their value. The s_nops are the wait states between a
+// VALU write and a DPP read of it.
+__device__ __forceinline__ float row_scan_product(float v) {
+  asm("s_nop 1\n\t"
+      "v_mul_f32_dpp %0, %0, %0 row_shr:1 row_mask:0xf bank_mask:0xf\n\t"
+      "s_nop 1\n\t"
+      "v_mul_f32_dpp %0, %0, %0 row_shr:2 row_mask:0xf bank_mask:0xf\n\t"
+      "s_nop 1\n\t"
+      "v_mul_f32_dpp %0, %0, %0 row_shr:4 row_mask:0xf bank_mask:0xf\n\t"
+      "s_nop 1\n\t"
+      "v_mul_f32_dpp %0, %0, %0 row_shr:8 row_mask:0xf bank_mask:0xf"
+      : "+v"(v));
+  return v;
+}
+__device__ __forceinline__ float row_scan_sum(float v) {
+  asm("s_nop 1\n\t"
+      "v_add_f32_dpp %0, %0, %0 row_shr:1 row_mask:0xf bank_mask:0xf\n\t"
+      "s_nop 1\n\t"
+      "v_add_f32_dpp %0, %0, %0 row_shr:2 row_mask:0xf bank_mask:0xf\n\t"
+      "s_nop 1\n\t"
+      "v_add_f32_dpp %0, %0, %0 row_shr:4 row_mask:0xf bank_mask:0xf\n\t"
+      "s_nop 1\n\t"
+      "v_add_f32_dpp %0, %0, %0 row_shr:8 row_mask:0xf bank_mask:0xf"
+      : "+v"(v));
+  return v;
+}
+// base + the scan of the lanes before this one in its row.
+__device__ __forceinline__ float row_before(float scan, float base) {
+  float r;
+  asm("s_nop 1\n\t"
+      "v_add_f32_dpp %0, %1, %2 row_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:0"
+      : "=v"(r)
+      : "v"(scan), "v"(base));
+  return r;
+}
+
+// Sums over the four DPP rows of a wave (lanes l, l ^ 16, l ^ 32, l ^ 48):
+// row r = lane >> 4 ends with values first(r) + j, j < ROW, of its 16
+// records, first(r) = (r >> 1) HALF + (r & 1) ROW.
+template <int N>
+struct RowSums {
+  static constexpr int HALF = (N + 1) / 2;
+  static constexpr int ROW = (HALF + 1) / 2;
+  static __device__ __forceinline__ void reduce(const float (&v)[N], float (&out)[ROW], int lane) {
+    float a[HALF];
+#pragma unroll
+    for (int j = 0; j < HALF; ++j)
+      a[j] = exchange_add<5>(v[j], j + HALF < N ? v[j + HALF] : 0.f, lane);
+#pragma unroll
+    for (int j = 0; j < ROW; ++j)
+      out[j] = exchange_add<4>(a[j], j + ROW < HALF ? a[j + ROW] : 0.f, lane);
+  }
+  static __device__ __forceinline__ int first(int row) {
+    return (row >> 1) * HALF + (row & 1) * ROW;
+  }
+  static __device__ __forceinline__ int count(int row) {
+    const int half = (row >> 1) ? N - HALF : HALF;  // real values in this half
+    return (row & 1) ? max(half - ROW, 0) : min(half, ROW);
+  }
+};
+
+// Compiler and LDS order between the lanes of one wave (LDS serves a wave's
+// accesses in order; nothing may move across).
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// One record's constants in a lane's registers.
+struct Record {
+  float row[15];  // what sample_surface reads: T 0-8, centre 9-10, normal 11-13, opacity 14
+  int position;   // list position, counted from 1
+  // Waves t_f = A_f s_u + B_f s_v + C_f (A_1 = B_1, A_3 = -B_3 and B_0 = 0 by
+  // their directions), weights, -2 pi HW_f A_f and B_f, and the colour's
+  // constant and factor.
+  float a0, a1, a2, b2, a3, c[4], hw[4], ap0, ap1, ap2, bp2, ap3, sumw[3], diff[3];
+};
+
+// Loads record `id` (appearance row and opacity of primitive `prim`) and
+// derives its constants; lanes without a record (present = false) take the
+// opacity 0, which no pixel accepts. (centre_x, centre_y) of the quadrant bound
+// the record's centre to kCentreReach pixels around it: further out no pixel of
+// the quadrant passes by rho2 (accepted samples have rho <= 2 ln(255 o) < 190 for
+// any float opacity, rho2 > 7000), so no decision changes, while the centre of a
+// surfel that crosses the camera plane can lie anywhere and would cost the moment
+// sums X and Y their precision. colour_sums (c1 + c2) is what only
+// record_gradients needs.
+constexpr float kCentreReach = 64.f;
+
+__device__ __forceinline__ void load_record(Record& rec, float* colour_sums, bool present,
+                                            int id, uint32_t prim, int position, float centre_x,
+                                            float centre_y, const float* __restrict__ geometry,
+                                            const float* __restrict__ appearance,
+                                            const float* __restrict__ opacities) {
+  const float* g = geometry + int64_t(id) * kGeometry;
+  const float* a = appearance + int64_t(prim) * kClassic;
+#pragma unroll
+  for (int i = 0; i < 14; ++i) rec.row[i] = g[i];
+  rec.row[9] = fminf(fmaxf(rec.row[9], centre_x - kCentreReach), centre_x + kCentreReach);
+  rec.row[10] = fminf(fmaxf(rec.row[10], centre_y - kCentreReach), centre_y + kCentreReach);
+  const float opacity = opacities[prim];
+  rec.row[14] = present ? opacity : 0.f;
+  rec.position = present ? position : INT_MAX;
+  const float m[4] = {a[10], a[11], a[12], a[13]};
+  rec.a0 = m[0] * kDirX[0];
+  rec.a1 = m[1] * kDirX[1];
+  rec.a2 = m[2] * kDirX[2];
+  rec.b2 = m[2] * kDirY[2];
+  rec.a3 = m[3] * kDirX[3];
+  float half_w = 0.f;
+#pragma unroll
+  for (int f = 0; f < 4; ++f) {
+    rec.c[f] = a[14 + f] * kInvTwoPi;
+    rec.hw[f] = 0.5f * a[6 + f];
+    half_w += rec.hw[f];
+  }
+  rec.ap0 = -kTwoPi * rec.hw[0] * rec.a0;
+  rec.ap1 = -kTwoPi * rec.hw[1] * rec.a1;
+  rec.ap2 = -kTwoPi * rec.hw[2] * rec.a2;
+  rec.bp2 = -kTwoPi * rec.hw[2] * rec.b2;
+  rec.ap3 = -kTwoPi * rec.hw[3] * rec.a3;
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    const float sum = a[c] + a[3 + c];
+    rec.sumw[c] = half_w * sum;
+    rec.diff[c] = a[c] - a[3 + c];
+    colour_sums[c] = sum;
+  }
+}
+
+// One step: this lane's record at its pixel `p` (ReplayPixel), whose state
+// (transmittance behind the chunk's records so far, running sum of w dL/dw)
+// is `state`; the summands are added into `sum`. Returns whether the pixel
+// took the record. Lanes that do not take it leave their exact zeros through
+// the stand-ins of sample_surface (see there); Masked also zeroes the
+// gradients of such lanes, for quadrants with a non-finite gradient or state.
+template <int Maps, bool Masked>
+__device__ __forceinline__ bool replay_step(const Record& rec, const float* p,
+                                            float2& state, float near_plane, float mscale,
+                                            float mnear, float* sum) {
+  using P = ReplayPixel;
+  using S = Sums<Maps>;
+  const float x = p[P::X], y = p[P::Y];
+  Sample v;
+  const bool active = sample_surface<false, true, false>(
+      rec.row, x, y, near_plane, rec.position <= __float_as_int(p[P::LAST]), v);
+  auto mask = [&](float t) { return Masked ? (active ? t : 0.f) : t; };
+  const float go[3] = {mask(p[P::RGB]), mask(p[P::RGB + 1]), mask(p[P::RGB + 2])};
+  const float alpha = v.alpha, inv_pz = v.inv_pz;
+  const float s[2] = {v.s[0], v.s[1]};
+  // Transmittance in front of the record: alpha = 0, inv_keep = 1 where the
+  // lane does not take it.
+  const float inv_keep = rcp(1.f - alpha);
+  const float T = state.x * row_scan_product(inv_keep);
+  const float w = T * alpha;
+  // dL/dw without the colour, and dL/dz / w (see the depth factors in
+  // renderBackward).
+  float gw = 0.f, g_depth = 0.f;
+  if constexpr (Maps >= kColourDepth) {
+    g_depth = mask(p[P::DEPTH]);
+    gw = g_depth * v.depth;
+  }
+  float gn[3];
+  if constexpr (Maps == kAllMaps) {
+    const float inv_depth = rcp(v.depth);
+    const float m = mscale - mnear * inv_depth;
+    gw += m * (mask(p[P::A8]) * m - mask(p[P::C8])) + mask(p[P::D8]);
+    g_depth += (mask(p[P::E8]) * m - mask(p[P::F8])) * (inv_depth * inv_depth);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      gn[c] = mask(p[P::NORMAL + c]);
+      gw += gn[c] * rec.row[11 + c];
+    }
+  }
+  float* app = sum + S::APPEARANCE;
+  float gs[2];
+  float t[4], cosine[4], sine[4];
+  t[0] = fract(fmaf(rec.a0, s[0], rec.c[0]));
+  t[1] = fract(fmaf(rec.a1, s[0], fmaf(rec.a1, s[1], rec.c[1])));
+  t[2] = fract(fmaf(rec.a2, s[0], fmaf(rec.b2, s[1], rec.c[2])));
+  t[3] = fract(fmaf(rec.a3, s[0], fmaf(-rec.a3, s[1], rec.c[3])));
+#pragma unroll
+  for (int f = 0; f < 4; ++f) {
+    cosine[f] = cos_rev(t[f]);
+    sine[f] = sin_rev(t[f]);
+  }
+  const float mix = rec.hw[0] * cosine[0] + rec.hw[1] * cosine[1] + rec.hw[2] * cosine[2] +
+                    rec.hw[3] * cosine[3];
+  const float dot_diff = go[0] * rec.diff[0] + go[1] * rec.diff[1] + go[2] * rec.diff[2];
+#pragma unroll
+  for (int c = 0; c < 3; ++c) gw += go[c] * rec.sumw[c];
+  gw += mix * dot_diff;
+  const float g_diff = w * dot_diff;
+  const float w_mix = w * mix;
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    app[c] += w * go[c];
+    app[3 + c] += w_mix * go[c];
+  }
+  // Along the waves' directions, the diagonal ones less their factor.
+  const float dot[4] = {s[0], s[0] + s[1], kDirX[2] * s[0] + kDirY[2] * s[1], s[1] - s[0]};
+  float gq[4];
+#pragma unroll
+  for (int f = 0; f < 4; ++f) {
+    gq[f] = sine[f] * g_diff;
+    app[6 + f] += cosine[f] * g_diff;
+    app[10 + f] += gq[f] * dot[f];
+    app[14 + f] += gq[f];
+  }
+  gs[0] = gq[0] * rec.ap0 + gq[1] * rec.ap1 + gq[2] * rec.ap2 + gq[3] * rec.ap3;
+  gs[1] = gq[1] * rec.ap1 + gq[2] * rec.bp2 - gq[3] * rec.ap3;
+  // Running sum behind the record, and the state in front of the chunk.
+  const float scan = row_scan_sum(w * gw);
+  const float galpha = mask(T * gw + (p[P::FINAL] - row_before(scan, state.y)) * inv_keep);
+  state.x = T;
+  state.y += scan;
+  if constexpr (Maps == kAllMaps) {
+#pragma unroll
+    for (int c = 0; c < 3; ++c) sum[S::NORMAL + c] += w * gn[c];
+  }
+  if constexpr (Maps >= kColourDepth) {
+    // The depth tilts with s only where the sample lies on the surface.
+    const float gz = w * g_depth;
+    const float gz_tilt = v.surface ? gz : 0.f;
+    gs[0] += gz_tilt * rec.row[6];
+    gs[1] += gz_tilt * rec.row[7];
+    sum[S::TILT + 0] += gz_tilt * s[0];
+    sum[S::TILT + 1] += gz_tilt * s[1];
+    sum[S::TILT + 2] += gz;
+  }
+  // alpha = min(0.99, o e) is below the clamp exactly when o e < 0.99.
+  const float ge = (active & (alpha < 0.99f)) ? galpha * v.e : 0.f;
+  sum[S::OPACITY] += ge;
+  // dL/drho = -o ge / 2; rho is rho3 = |s|^2 on the surface (d/ds = 2 s) and
+  // otherwise rho2 = 2 |centre - pixel|^2 (d/dcentre = 4 (centre - pixel)):
+  // grho2 is half the latter's factor, the rest is left to record_gradients.
+  const float g2 = -rec.row[14] * ge;
+  const float grho3 = v.surface ? g2 : 0.f;
+  const float grho2 = v.surface ? 0.f : g2;
+  gs[0] += s[0] * grho3;
+  gs[1] += s[1] * grho3;
+  const float dx = rec.row[9] - x, dy = rec.row[10] - y;
+  sum[S::XY + 0] += dx * grho2;
+  sum[S::XY + 1] += dy * grho2;
+  const float gp0 = gs[0] * inv_pz, gp1 = gs[1] * inv_pz;
+  const float gp[3] = {gp0, gp1, -(gp0 * s[0] + gp1 * s[1])};
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    sum[S::G + k] += gp[k];
+    sum[S::X + k] += dx * gp[k];
+    sum[S::Y + k] += dy * gp[k];
+  }
+  return active;
+}
+
+__device__ __forceinline__ void cross(const float* a, const float* b, float* out) {
+  out[0] = a[1] * b[2] - a[2] * b[1];
+  out[1] = a[2] * b[0] - a[0] * b[2];
+  out[2] = a[0] * b[1] - a[1] * b[0];
+}
+
+// A record's output gradients from its sums, in place: geometry columns 0..13,
+// appearance columns, opacity.
+//  With T0c = T0 - cx T2, T1c = T1 - cy T2 about the record's centre (cx, cy),
+//  k = -dx T2 - T0c and l = -dy T2 - T1c, so that (sums over the pixels)
+//    sum gp x l = -Y x T2 - G x T1c                    -> dT0
+//    sum k x gp = -T2 x X - T0c x G                    -> dT1
+//    sum x (gp x l) + y (k x gp) = cx dT0 + cy dT1 + X x T1c + T0c x Y,
+//  the negative of which, with the depth's TILT, is dT2 (the terms in dx dy
+//  cancel). colour_sums: c1 + c2.
+template <int Maps>
+__device__ __forceinline__ void record_gradients(const Record& rec, const float* colour_sums,
+                                                 float* out) {
+  using S = Sums<Maps>;
+  float v[S::COUNT];
+#pragma unroll
+  for (int i = 0; i < S::COUNT; ++i) v[i] = out[i];
+  const float* t2 = rec.row + 6;
+  const float cx = rec.row[9], cy = rec.row[10];
+  float t0[3], t1[3];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    t0[k] = rec.row[k] - cx * t2[k];
+    t1[k] = rec.row[3 + k] - cy * t2[k];
+  }
+  float y_t2[3], g_t1[3], t2_x[3], t0_g[3], x_t1[3], t0_y[3];
+  cross(v + S::Y, t2, y_t2);
+  cross(v + S::G, t1, g_t1);
+  cross(t2, v + S::X, t2_x);
+  cross(t0, v + S::G, t0_g);
+  cross(v + S::X, t1, x_t1);
+  cross(t0, v + S::Y, t0_y);
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const float d0 = -y_t2[k] - g_t1[k], d1 = -t2_x[k] - t0_g[k];
+    out[k] = d0;
+    out[3 + k] = d1;
+    const float tilt = Maps >= kColourDepth ? v[S::TILT + k] : 0.f;
+    out[6 + k] = tilt - (cx * d0 + cy * d1 + x_t1[k] + t0_y[k]);
+  }
+  out[9] = 2.f * v[S::XY];
+  out[10] = 2.f * v[S::XY + 1];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) out[11 + k] = Maps == kAllMaps ? v[S::NORMAL + k] : 0.f;
+  const float* app = v + S::APPEARANCE;
+  // colour_c = W/2 SUM_c + S DIFF_c, S = sum_f HW_f cos_f, W/2 = sum_f HW_f.
+  float* to = out + 14;
+  const float half_w = rec.hw[0] + rec.hw[1] + rec.hw[2] + rec.hw[3];
+  float g_sum = 0.f;
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    to[c] = half_w * app[c] + app[3 + c];
+    to[3 + c] = half_w * app[c] - app[3 + c];
+    g_sum += colour_sums[c] * app[c];
+  }
+#pragma unroll
+  for (int f = 0; f < 4; ++f) {
+    const float along = f & 1 ? kDirY[f] : 1.f;  // the diagonal waves' factor
+    to[6 + f] = 0.5f * (g_sum + app[6 + f]);
+    to[10 + f] = -kTwoPi * along * rec.hw[f] * app[10 + f];
+    to[14 + f] = -rec.hw[f] * app[14 + f];
+  }
+  to[kClassic] = v[S::OPACITY];
+}
+
+constexpr int kGeometryOut = 14;                        // geometry columns written
+constexpr int kOutputs = kGeometryOut + kClassic + 1;  // per record
+constexpr int kSumPitch = 37;  // a record's sums, then its outputs in their place
+static_assert(kSumPitch >= kOutputs && kSumPitch >= Sums<kAllMaps>::COUNT, "a record's LDS row");
+
+struct Wave {
+  float pixels[64 * ReplayPixel::FLOATS];
+  float2 state[64];
+  // The chunk's sums; during the walk, where lanes without a state to keep
+  // write theirs.
+  float sums[kChunk * kSumPitch];
+  float colour_sums[kChunk * 3];
+  uint64_t rows[kChunk][2];  // the gradient rows of the chunk's records
+  int ids[kQueue];
+  uint32_t prims[kQueue];
+  int positions[kQueue];
+};
+
+// The replay walk's backward compositor: one workgroup per tile, or per
+// segment of a split tile (`segments`), one wave per quadrant.
+template <int Maps>
+__global__ __launch_bounds__(kTilePixels, 3) void renderBackward(
+    int width, int height, int tw, int th, const float* __restrict__ geometry,
+    const float* __restrict__ appearance, const float* __restrict__ opacities,
+    const int64_t* __restrict__ primitive_ids, const float* __restrict__ backgrounds,
+    const int2* __restrict__ ranges, const int* __restrict__ order,
+    const int2* __restrict__ replay, const int* __restrict__ replay_counts,
+    const float* __restrict__ state, const int* __restrict__ contributors,
+    MapGroups<const float> grad_maps, float near_plane, float far_plane,
+    float* __restrict__ grad_geometry, float* __restrict__ grad_appearance,
+    float* __restrict__ grad_opacities, float* __restrict__ grad_backgrounds,
+    const int2* __restrict__ segments, Segments seg) {
+  using S = Sums<Maps>;
+  using P = ReplayPixel;
+  __shared__ __align__(16) Wave waves[kTilePixels / 64];
+  __shared__ float bg_acc[3];
+  const int lane = lane_id();
+  // (tile, segment) of this workgroup; past the segment count: nothing.
+  const int2 piece = segments ? segments[blockIdx.x] : make_int2(order[blockIdx.x], 0);
+  if (piece.x < 0) return;
+  const int tile = piece.x;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  Wave& lds = waves[wave];
+#ifdef GS_DIAGNOSTICS
+  const long long diag_begin = wall_clock64();
+  __shared__ unsigned int diag_lanes[65];
+  __shared__ unsigned int diag_packing[5];
+  for (int i = threadIdx.x; i < 65; i += kTilePixels) diag_lanes[i] = 0u;
+  if (threadIdx.x < 5) diag_packing[threadIdx.x] = 0u;
+  PackingCounts packing;
+#endif
+  if (threadIdx.x < 3) bg_acc[threadIdx.x] = 0.f;
+  // Per pixel (one per lane): its gradients and final state, staged for the
+  // steps.
+  const TilePixel tp = tile_pixel(tile, width, height, tw, th);
+  float go[kMaps];
+#pragma unroll
+  for (int c = 0; c < kMaps; ++c) {
+    const float* g = grad_maps.data[map_group(c)];  // null: no gradient for the group
+    go[c] = (tp.inside && g) ? g[grad_maps.offset(c, tp.pixel)] : 0.f;
+  }
+  const float final_t = tp.inside ? state[tp.pixel * 3 + 0] : 0.f;
+  const float m1 = tp.inside ? state[tp.pixel * 3 + 1] : 0.f;
+  const float m2 = tp.inside ? state[tp.pixel * 3 + 2] : 0.f;
+  const float total_a = 1.f - final_t;
+  float T = final_t;
+  float background_dot = 0.f;
+#pragma unroll
+  for (int c = 0; c < 3; ++c) background_dot += go[c] * backgrounds[tp.image * 3 + c];
+  // dL/dalpha_i picks up final_t (go_alpha - background . go_rgb) / (1 - alpha_i).
+  const float final_term = final_t * (go[3] - background_dot);
+  // The replay entries [block_first, block_last) of the tile: all of them, or
+  // one segment's of a split tile, which starts from checkpoint c_{k+1}: its
+  // transmittance, and the suffix sum_{later records} w dL/dw from
+  // c_K - c_{k+1} (the map gradients weigh the prefix-sum differences;
+  // distortion through the final m1, m2).
+  const int2 range = ranges[tile];
+  int block_first = 0, block_last = replay_counts[tile];
+  float suffix = 0.f;
+  if (seg.length > 0 && seg.index[tile] >= 0) {
+    const int base = seg.index[tile];
+    const int pieces = segment_count(range.y - range.x, seg.length);
+    const int* n = seg.index + seg.tiles + base;
+    block_first = piece.y ? n[piece.y - 1] : 0;
+    block_last = n[piece.y];
+    if (piece.y < pieces - 1 && tp.inside) {
+      constexpr int kSlot = kCheckpointFloats * kTilePixels;
+      const float* c = seg.state + int64_t(base + piece.y) * kSlot + threadIdx.x;
+      const float* f = seg.state + int64_t(base + pieces - 1) * kSlot + threadIdx.x;
+      float d[10];  // T, rgb, depth, normals, m1, m2
+#pragma unroll
+      for (int q = 0; q < 10; ++q) d[q] = f[q * kTilePixels] - c[q * kTilePixels];
+      T = c[0];
+      suffix = go[0] * d[1] + go[1] * d[2] + go[2] * d[3] + go[4] * d[4] + go[5] * d[5] +
+               go[6] * d[6] + go[7] * d[7] +
+               go[8] * (total_a * d[9] - m2 * d[0] - 2.f * m1 * d[8]);
+    }
+  }
+  // Whether every map gradient and saved state value of the quadrant's pixels
+  // is finite (selects the step without per-lane masking).
+  bool finite = isfinite(final_term) && isfinite(m1) && isfinite(m2) && isfinite(T) &&
+                isfinite(suffix);
+#pragma unroll
+  for (int c = 0; c < kMaps; ++c) finite = finite && isfinite(go[c]);
+  const bool finite_pixels = __all(finite);
+  const float mscale = far_plane / (far_plane - near_plane);
+  const float mnear = mscale * near_plane;
+  {
+    // Depth and distortion factors, with g4, g8 their map gradients and
+    // A = 1 - final T:
+    //   g4 depth + g8 (m^2 A + m2 - 2 m m1) = g4 depth + m (a8 m - c8) + d8,
+    //   dL/dz = w g4 + 2 w g8 mnear (m A - m1) / depth^2
+    //         = w (g4 + (e8 m - f8) / depth^2),
+    // a8 = g8 A, c8 = 2 g8 m1, d8 = g8 m2, e8 = 2 a8 mnear, f8 = c8 mnear.
+    const float a8 = go[8] * total_a, c8 = 2.f * go[8] * m1, d8 = go[8] * m2;
+    float4* p = reinterpret_cast<float4*>(lds.pixels + lane * P::FLOATS);
+    // Outside the image last = 0: no record's position (from 1) is within it.
+    const int last = tp.inside ? contributors[tp.pixel] : 0;
+    p[0] = make_float4(go[0], go[1], go[2], go[5]);
+    p[1] = make_float4(go[6], go[7], float(tp.px), float(tp.py));
+    p[2] = make_float4(__int_as_float(last), final_term, go[4], a8);
+    p[3] = make_float4(c8, d8, 2.f * a8 * mnear, c8 * mnear);
+    lds.state[lane] = make_float2(T, suffix);
+  }
+  __syncthreads();
+  // Background gradient: sum over the tile of final T * dL/drgb (once per
+  // tile: by its first segment).
+  if (piece.y == 0) {
+    const float gb[3] = {final_t * go[0], final_t * go[1], final_t * go[2]};
+    const float total = wave_reduce_quads<3>(gb, lane);
+    const int param = rs_quad_param<3>(lane);
+    if (param < 3 && total != 0.f) atomicAdd(&bg_acc[param], total);
+  }
+  __syncthreads();
+  if (threadIdx.x < 3 && bg_acc[threadIdx.x] != 0.f)
+    atomicAdd(grad_backgrounds + tp.image * 3 + threadIdx.x, bg_acc[threadIdx.x]);
+
+  const int slot = lane & (kChunk - 1), row = lane >> 4;
+  auto uniform = [](float v) {
+    return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
+  };
+  const float centre_x = uniform(float(tp.px - (lane & 7)) + 3.5f);
+  const float centre_y = uniform(float(tp.py - (lane >> 3)) + 3.5f);
+  const int quadrant = kReplayPositionBits + wave;
+  // Lane 15 of a row keeps its pixel's state, the others write theirs aside.
+  float2* const aside = reinterpret_cast<float2*>(lds.sums);
+  float2* const state_row = (slot == kChunk - 1 ? lds.state : aside) + row;
+  static_assert(kChunk * kSumPitch >= 2 * 64, "the sums hold a quadrant's states");
+
+  auto walk_chunks = [&](auto masked) {
+    constexpr bool kMasked = decltype(masked)::value;
+    int head = 0, tail = 0;  // ring positions: queued entries are [head, tail)
+    int next = block_last;   // entries [block_first, next) are still to be read
+    // Entry read ahead of the wave's next 64.
+    int2 ahead = make_int2(0, 0);
+    if (next - 1 - lane >= block_first) ahead = replay[range.x + next - 1 - lane];
+    while (true) {
+      // Queue the quadrant's entries until a chunk is full or none are left.
+      while (tail - head < kChunk && next > block_first) {
+        const bool keep = next - 1 - lane >= block_first && ((uint32_t(ahead.y) >> quadrant) & 1u);
+        const uint64_t kept = __ballot(keep);
+        if (keep) {
+          const int before = int(__builtin_amdgcn_mbcnt_hi(
+              uint32_t(kept >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(kept), 0u)));
+          const int at = (tail + before) & (kQueue - 1);
+          lds.ids[at] = ahead.x;
+          lds.positions[at] = (ahead.y & kReplayPositionMask) + 1;
+          lds.prims[at] = uint32_t(primitive_ids[ahead.x]);
+        }
+        tail += __popcll(kept);
+        next -= 64;
+        if (next - 1 - lane >= block_first) ahead = replay[range.x + next - 1 - lane];
+      }
+      const int n = min(kChunk, tail - head);
+      if (n <= 0) break;
+      wave_lds_fence();
+      const int at = (head + min(slot, n - 1)) & (kQueue - 1);
+      const int id = lds.ids[at];
+      const uint32_t prim = lds.prims[at];
+      head += n;
+      Record rec;
+      float colour_sums[3];
+      load_record(rec, colour_sums, slot < n, id, prim, lds.positions[at], centre_x, centre_y,
+                          geometry, appearance, opacities);
+      auto address = [](const float* t) { return reinterpret_cast<uint64_t>(t); };
+      if (row == 0) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) lds.colour_sums[slot * 3 + c] = colour_sums[c];
+        lds.rows[slot][0] = address(grad_geometry) + uint64_t(int64_t(id) * kGeometry) * 4;
+        lds.rows[slot][1] =
+            address(grad_appearance) + uint64_t(prim) * (kClassic * 4) - kGeometryOut * 4;
+      }
+      float sum[S::COUNT];
+#pragma unroll
+      for (int i = 0; i < S::COUNT; ++i) sum[i] = 0.f;
+#ifdef GS_DIAGNOSTICS
+      uint64_t took = 0;
+#endif
+#pragma unroll 1
+      for (int g = 0; g < kGroups; ++g) {
+        const int q = 4 * g + row;
+        float p[P::FLOATS];
+        const float4* from = reinterpret_cast<const float4*>(lds.pixels + q * P::FLOATS);
+#pragma unroll
+        for (int i = 0; i < P::FLOATS / 4; ++i) {
+          const float4 t = from[i];
+          p[4 * i] = t.x;
+          p[4 * i + 1] = t.y;
+          p[4 * i + 2] = t.z;
+          p[4 * i + 3] = t.w;
+        }
+        float2 st = lds.state[q];
+        const bool active = replay_step<Maps, kMasked>(rec, p, st, near_plane, mscale, mnear, sum);
+        (void)active;
+#ifdef GS_DIAGNOSTICS
+        if (active) took |= uint64_t(1) << q;
+#endif
+        state_row[4 * g] = st;
+      }
+#ifdef GS_DIAGNOSTICS
+      took |= __shfl_xor(took, 16, 64);
+      took |= __shfl_xor(took, 32, 64);
+      for (int j = 0; j < n; ++j) {
+        const uint64_t taking = __shfl(took, j, 64);
+        if (lane == 0 && taking) atomicAdd(&diag_lanes[__popcll(taking)], 1u);
+        if (taking) packing.add(taking);
+      }
+      packing.flush(diag_packing);
+#endif
+      wave_lds_fence();
+      // The record's sums over the four pixel rows, then its gradients.
+      {
+        using R = RowSums<S::COUNT>;
+        float part[R::ROW];
+        R::reduce(sum, part, lane);
+        float* to = lds.sums + slot * kSumPitch + R::first(row);
+        const int count = R::count(row);
+#pragma unroll
+        for (int j = 0; j < R::ROW; ++j)
+          if (j < count) to[j] = part[j];
+      }
+      wave_lds_fence();
+      if (lane < n) {
+        float* out = lds.sums + lane * kSumPitch;
+        record_gradients<Maps>(rec, lds.colour_sums + lane * 3, out);
+      }
+      wave_lds_fence();
+      // One global atomic per nonzero output; consecutive lanes take
+      // consecutive columns of a record, so that a wave's atomics fall on a few
+      // cache lines.
+      // Half a wave per record: columns 0..13 geometry, 14..31 appearance.
+      static_assert(kOutputs == 33, "32 columns and the opacity");
+      const int p = lane & 31, half = lane >> 5;
+      const uint64_t* base = &lds.rows[half][p >= kGeometryOut];
+      const float* value = lds.sums + half * kSumPitch + p;
+#pragma unroll
+      for (int j = 0; j < kChunk; j += 2) {
+        const float v = value[j * kSumPitch];
+        if (j + half < n && v != 0.f) global_add(base[2 * j] + p * 4, v);
+      }
+      if (lane < n) {
+        const float v = lds.sums[lane * kSumPitch + 32];
+        if (v != 0.f) global_add(address(grad_opacities + prim), v);
+      }
+      // The ring's consumed slots and the sums may be overwritten from here on.
+      wave_lds_fence();
+    }
+  };
+  if (finite_pixels)
+    walk_chunks(std::false_type{});
+  else
+    walk_chunks(std::true_type{});
+#ifdef GS_DIAGNOSTICS
+  __syncthreads();
+  if (gs_diagnostics.lanes && threadIdx.x < 65 && diag_lanes[threadIdx.x] != 0u)
+    atomicAdd(gs_diagnostics.lanes + threadIdx.x,
+              static_cast<unsigned long long>(diag_lanes[threadIdx.x]));
+  if (gs_diagnostics.counters && threadIdx.x < 5 && diag_packing[threadIdx.x] != 0u)
+    atomicAdd(gs_diagnostics.counters + 2 + threadIdx.x,
+              static_cast<unsigned long long>(diag_packing[threadIdx.x]));
+  stamp_tile(gs_diagnostics.backward_span, tile, diag_begin);
+#endif
+}
+
+}  // namespace by_record
 
 struct RenderWorkspace {
   int* order;      // [tiles]
@@ -2513,19 +3196,29 @@ int gs_render_backward(int32_t neural, const float* geometry, const float* appea
     GS_LAUNCHED("tile_order_kernel");
   }
   const int2* lists = reinterpret_cast<const int2*>(replay);
-  auto launch = [&](auto kernel) {
-    kernel<<<blocks, kTilePixels, 0, s>>>(
-        width, height, tw, th, geometry, appearance, opacities, primitive_ids, backgrounds,
-        point_list, r, w.order, w.tile_last, lists, replay_counts, state, contributors, grads,
-        near_plane, far_plane, grad_geometry, grad_rows, grad_opacities,
-        grad_backgrounds, w.segments, seg);
-  };
-  if (neural) {
-    if (replay) launch(renderBackward<true, true>);
-    else launch(renderBackward<true, false>);
+  if (replay && !neural) {
+    auto launch = [&](auto kernel) {
+      kernel<<<blocks, kTilePixels, 0, s>>>(
+          width, height, tw, th, geometry, appearance, opacities, primitive_ids, backgrounds, r,
+          w.order, lists, replay_counts, state, contributors, grads, near_plane, far_plane,
+          grad_geometry, grad_appearance, grad_opacities, grad_backgrounds, w.segments, seg);
+    };
+    // The step leaves out what the absent gradient groups would feed
+    // (by_record::renderBackward).
+    if (grad_maps[3] || grad_maps[4]) launch(by_record::renderBackward<by_record::kAllMaps>);
+    else if (grad_maps[2]) launch(by_record::renderBackward<by_record::kColourDepth>);
+    else launch(by_record::renderBackward<by_record::kColour>);
   } else {
-    if (replay) launch(renderBackward<false, true>);
-    else launch(renderBackward<false, false>);
+    auto launch = [&](auto kernel) {
+      kernel<<<blocks, kTilePixels, 0, s>>>(
+          width, height, tw, th, geometry, appearance, opacities, primitive_ids, backgrounds,
+          point_list, r, w.order, w.tile_last, lists, replay_counts, state, contributors, grads,
+          near_plane, far_plane, grad_geometry, grad_rows, grad_opacities,
+          grad_backgrounds, w.segments, seg);
+    };
+    if (!neural) launch(renderBackward<false, false>);
+    else if (replay) launch(renderBackward<true, true>);
+    else launch(renderBackward<true, false>);
   }
   GS_LAUNCHED("renderBackward");
   return GS_OK;
