@@ -292,34 +292,39 @@ __global__ __launch_bounds__(kSortBlock) void radix_downsweep_kernel(
 }
 
 // Sorts of up to kLocalSort keys run in one workgroup of kLocalBlock
-// threads, every pass in one launch: each thread keeps kLocalItems keys in
-// registers (key i of wave w is item (i - w 64 kLocalItems) / 64 of lane
-// i mod 64, so a wave's keys are ranked in order, as in the downsweep), the
-// per-wave digit counters give every key its slot, and between passes the
-// keys are restaged through LDS; the last pass writes the output.
+// threads, every pass in one launch: each thread keeps Items keys in
+// registers (key i of wave w is item (i - w 64 Items) / 64 of lane i mod 64,
+// so a wave's keys are ranked in order, as in the downsweep), the per-wave
+// digit counters give every key its slot, and between passes the keys are
+// restaged through LDS; the last pass writes the output. One workgroup's
+// latency bounds it: Items is the fewest that hold the keys, so that all
+// waves rank (an item costs a ballot per digit bit), and digits are as wide
+// as in the multi-workgroup passes. 1024 depth keys of 27 bits, with eight
+// items in two waves and four passes 25.6 us, with one item and three passes
+// 8.3 us.
 constexpr int kLocalBlock = 1024;
 constexpr int kLocalWaves = kLocalBlock / 64;
 constexpr int kLocalItems = 8;
 constexpr int64_t kLocalSort = int64_t(kLocalBlock) * kLocalItems;
 
-template <typename Key, bool Values>
+template <typename Key, bool Values, int Items, int Bins>
 __global__ __launch_bounds__(kLocalBlock) void local_sort_kernel(
     const Key* __restrict__ keys_in, const int* __restrict__ values_in,
     Key* __restrict__ keys_out, int* __restrict__ values_out, int64_t capacity,
     const int64_t* __restrict__ live, int begin_bit, int end_bit, int passes, int digit_bits) {
   const int m = int(live_length(capacity, live));
-  __shared__ uint32_t running[kLocalWaves][kBins];  // per-wave digit counters
-  __shared__ uint32_t digit_start[kBins];
-  __shared__ uint32_t wave_totals[kBins / 64];
-  __shared__ Key stage_keys[kLocalSort];
-  __shared__ int stage_values[Values ? kLocalSort : 1];
+  __shared__ uint32_t running[kLocalWaves][Bins];  // per-wave digit counters
+  __shared__ uint32_t digit_start[Bins];
+  __shared__ uint32_t wave_totals[Bins / 64];
+  __shared__ Key stage_keys[kLocalBlock * Items];
+  __shared__ int stage_values[Values ? kLocalBlock * Items : 1];
   const int lane = __lane_id(), wave = threadIdx.x >> 6;
-  const int wave_base = wave * 64 * kLocalItems;
+  const int wave_base = wave * 64 * Items;
   const uint64_t lanes_below = (uint64_t(1) << lane) - 1;
-  Key key[kLocalItems];
-  int value[kLocalItems];
+  Key key[Items];
+  int value[Items];
 #pragma unroll
-  for (int it = 0; it < kLocalItems; ++it) {
+  for (int it = 0; it < Items; ++it) {
     const int i = wave_base + it * 64 + lane;
     key[it] = i < m ? keys_in[i] : Key(0);
     value[it] = Values && i < m ? values_in[i] : 0;
@@ -328,13 +333,13 @@ __global__ __launch_bounds__(kLocalBlock) void local_sort_kernel(
     const int shift = begin_bit + pass * digit_bits;
     const int bits = min(digit_bits, end_bit - shift);
     const uint32_t mask = (1u << bits) - 1u;
-    for (int i = threadIdx.x; i < kLocalWaves * kBins; i += kLocalBlock)
+    for (int i = threadIdx.x; i < kLocalWaves * Bins; i += kLocalBlock)
       (&running[0][0])[i] = 0;
     __syncthreads();
-    uint32_t rank[kLocalItems], before[kLocalItems];
-    int leader[kLocalItems];
+    uint32_t rank[Items], before[Items];
+    int leader[Items];
 #pragma unroll
-    for (int it = 0; it < kLocalItems; ++it) {
+    for (int it = 0; it < Items; ++it) {
       const bool valid = wave_base + it * 64 + lane < m;
       const uint32_t digit = uint32_t(key[it] >> shift) & mask;
       const uint64_t peers = digit_peers(digit, valid, bits);
@@ -345,25 +350,27 @@ __global__ __launch_bounds__(kLocalBlock) void local_sort_kernel(
         before[it] = atomicAdd(&running[wave][digit], uint32_t(__popcll(peers)));
     }
 #pragma unroll
-    for (int it = 0; it < kLocalItems; ++it)
+    for (int it = 0; it < Items; ++it)
       rank[it] += uint32_t(__shfl(int(before[it]), leader[it]));
     __syncthreads();
     // Per digit: each wave's first slot among the digit's keys, the
-    // digit's total, then the exclusive prefix over digits (waves 0-3).
-    if (threadIdx.x < kBins) {
+    // digit's total, then the exclusive prefix over digits (the first waves).
+    if (threadIdx.x < Bins) {
       const int d = threadIdx.x;
-      uint32_t run = 0;
+      uint32_t c[kLocalWaves], run = 0;
+#pragma unroll
+      for (int w = 0; w < kLocalWaves; ++w) c[w] = running[w][d];
+#pragma unroll
       for (int w = 0; w < kLocalWaves; ++w) {
-        const uint32_t c = running[w][d];
         running[w][d] = run;
-        run += c;
+        run += c[w];
       }
       const uint32_t incl = wave_inclusive_scan(run);
       if (lane == 63) wave_totals[wave] = incl;
       digit_start[d] = incl - run;
     }
     __syncthreads();
-    if (threadIdx.x < kBins) {
+    if (threadIdx.x < Bins) {
       uint32_t below = 0;
       for (int w = 0; w < wave; ++w) below += wave_totals[w];
       digit_start[threadIdx.x] += below;
@@ -371,7 +378,7 @@ __global__ __launch_bounds__(kLocalBlock) void local_sort_kernel(
     __syncthreads();
     const bool last = pass == passes - 1;
 #pragma unroll
-    for (int it = 0; it < kLocalItems; ++it) {
+    for (int it = 0; it < Items; ++it) {
       const int i = wave_base + it * 64 + lane;
       if (i < m) {
         const uint32_t digit = uint32_t(key[it] >> shift) & mask;
@@ -390,7 +397,7 @@ __global__ __launch_bounds__(kLocalBlock) void local_sort_kernel(
     if (!last) {
       __syncthreads();
 #pragma unroll
-      for (int it = 0; it < kLocalItems; ++it) {
+      for (int it = 0; it < Items; ++it) {
         const int i = wave_base + it * 64 + lane;
         key[it] = i < m ? stage_keys[i] : Key(0);
         value[it] = Values && i < m ? stage_values[i] : 0;
@@ -467,16 +474,6 @@ int radix_sort(const Key* keys_in, Key* keys_out, const int* values_in, int* val
     GS_LAUNCHED("copy_pairs_kernel");
     return GS_OK;
   }
-  if (m <= kLocalSort) {
-    auto local = [&](auto kernel) {
-      kernel<<<1, kLocalBlock, 0, s>>>(keys_in, values_in, keys_out, values_out, m, live,
-                                       begin_bit, end_bit, passes, digit_bits);
-    };
-    if (values_in) local(local_sort_kernel<Key, true>);
-    else local(local_sort_kernel<Key, false>);
-    GS_LAUNCHED("local_sort_kernel");
-    return GS_OK;
-  }
   // Wider digits for 32-bit keys when they save a pass.
   if (sizeof(Key) == 4) {
     const int wide_passes = int(ceil_div(bits_total, kWideDigitBits));
@@ -486,6 +483,27 @@ int radix_sort(const Key* keys_in, Key* keys_out, const int* values_in, int* val
     }
   }
   const int bins = digit_bits <= kDigitBits ? kBins : kWideBins;
+  if (m <= kLocalSort) {
+    auto local = [&](auto items_tag, auto bins_tag) {
+      constexpr int I = decltype(items_tag)::value, B = decltype(bins_tag)::value;
+      auto launch = [&](auto kernel) {
+        kernel<<<1, kLocalBlock, 0, s>>>(keys_in, values_in, keys_out, values_out, m, live,
+                                         begin_bit, end_bit, passes, digit_bits);
+      };
+      if (values_in) launch(local_sort_kernel<Key, true, I, B>);
+      else launch(local_sort_kernel<Key, false, I, B>);
+    };
+    auto by_length = [&](auto bins_tag) {
+      if (m <= kLocalBlock) local(std::integral_constant<int, 1>{}, bins_tag);
+      else if (m <= 2 * kLocalBlock) local(std::integral_constant<int, 2>{}, bins_tag);
+      else if (m <= 4 * kLocalBlock) local(std::integral_constant<int, 4>{}, bins_tag);
+      else local(std::integral_constant<int, kLocalItems>{}, bins_tag);
+    };
+    if (bins == kBins) by_length(std::integral_constant<int, kBins>{});
+    else by_length(std::integral_constant<int, kWideBins>{});
+    GS_LAUNCHED("local_sort_kernel");
+    return GS_OK;
+  }
   // Ping-pong so that the last pass writes the caller's output.
   const Key* src_k = keys_in;
   const int* src_v = values_in;

@@ -63,6 +63,25 @@ def test_sort32_is_stable_radix_order(native, m, bits, with_values):
         assert sv is None
 
 
+@pytest.mark.parametrize("m", [63, 64, 65, 1023, 1024, 1025, 2047, 4096, 4097, 8191])
+@pytest.mark.parametrize("bits, with_values", [((5, 32), True), ((0, 27), False), ((0, 8), True)])
+def test_local_sort_items(native, m, bits, with_values):
+    """The one-workgroup sort at the edges of its keys per thread (1, 2, 4 and
+    8), with 9-bit digits (27 bits in three passes) and 8-bit ones."""
+    rng = np.random.default_rng(m)
+    keys = rng.integers(0, 2**32, m, dtype=np.uint64).astype(np.uint32)
+    keys[m // 2:] = keys[: m - m // 2]  # ties across waves
+    values = np.arange(m, dtype=np.int32)[::-1].copy()
+    sk, sv = native.sort_pairs32(torch.from_numpy(keys.view(np.int32)).to(DEVICE),
+                                 torch.from_numpy(values).to(DEVICE) if with_values else None,
+                                 *bits)
+    digit = (keys >> np.uint32(bits[0])) & np.uint32((1 << (bits[1] - bits[0])) - 1)
+    order = np.argsort(digit, kind="stable")
+    np.testing.assert_array_equal(sk.cpu().numpy().view(np.uint32), keys[order])
+    if with_values:
+        np.testing.assert_array_equal(sv.cpu().numpy(), values[order])
+
+
 @pytest.mark.parametrize("m", [1, 5, 4095, 4096, 4097, 8192, 8193, 100_003, 2_000_000])
 @pytest.mark.parametrize("bits", [(0, 64), (0, 45), (32, 45), (3, 17)])
 def test_sort_is_stable_radix_order(native, m, bits):
