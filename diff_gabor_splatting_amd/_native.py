@@ -40,7 +40,9 @@ REPLAY_MAX_ENTRIES = 2**28 - 1
 # Split tiles (gs_render_forward's segment_* arguments): images with fewer
 # tiles than SPLIT_MAX_TILES have too few workgroups to hide a long tile
 # list, so tiles longer than SPLIT_LENGTH records are composited (and their
-# backward replayed) in segments of that many records, one workgroup each.
+# backward replayed) in segments of that many records, one workgroup each;
+# beyond 256 tiles only where that pays, which the forward decides on the
+# device from the longest list and the number of segments.
 # The segment length does not depend on the intersection count, and the
 # checkpoint slots are at most SPLIT_MAX_SLOTS, so a render into a
 # fixed-capacity point list splits its tiles exactly as the synchronised

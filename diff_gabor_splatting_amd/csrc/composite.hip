@@ -822,7 +822,7 @@ __device__ __forceinline__ int append_replay(const uint64_t* wave_taken, const i
 
 // Split tiles. A tile whose point list is longer than `length` records (a
 // multiple of kBatch) is replayed by the backward in segments, one
-// workgroup each: segment k takes the replay entries the forward appended
+// workgroup each, unless the image's tiles are walked whole (whole_pays): segment k takes the replay entries the forward appended
 // while walking list records [k length, (k + 1) length). For it the forward
 // writes checkpoints c_1 .. c_K (K = ceil(list length / length)): c_j is the
 // per-pixel prefix state after the first j length records (c_K: the final
@@ -967,25 +967,64 @@ __device__ __forceinline__ int block_inclusive_sum(int v, int* wave_totals, int*
   return before + incl;
 }
 
+// Whether a split render's long tiles are walked whole after all, from the
+// longest list and the number of segments. Up to kSplitAllTiles tiles (about
+// one workgroup per CU) they are split: the segments run on CUs that would
+// idle. Beyond, the segments compete for CUs that are busy anyway, walk records
+// behind the pixels' stops and pay a merge that grows with their number, while
+// splitting saves the walk of the longest list. One long list among short ones
+// decides the length of the whole launch, so all tiles are split or none. The
+// lines are the ratios of both at which the times of 45 scenes of 256 to 2,016
+// tiles part, forward and backward together, split against whole: 640x480 of
+// 30k surfels (longest 227, 3,773 segments) 300 against 241 us, four 256x256
+// views of 10k (372, 3,095) 270 and 226, longest 967 of 7,142 segments 530 and
+// 303, but 1,080 of 3,245 384 and 454, 588 of 1,631 242 and 292. Neural: 328 of
+// 3,468 372 and 320, 1,176 of 11,730 1,227 and 656, but 370 of 3,106 383 and
+// 417, 783 of 3,983 536 and 678. The rule reads the lists on the device, so a
+// fixed-capacity render decides as the synchronised one does.
+constexpr int kSplitAllTiles = 256;
+
+__device__ __forceinline__ bool whole_pays(bool neural, int longest, int segments) {
+  return longest <= (neural ? segments / 7 - 100 : max(segments / 5, 170));
+}
+
 // cost: per-tile cost, or null to use the tile's list length from ranges.
-// With seg.length > 0 (the forward of split tiles) it also assigns each
-// tile longer than seg.length its ceil(length / seg.length) checkpoint
+// With seg.length > 0 (the forward of split tiles) it writes the (tile,
+// segment) work list in place of `order`, and assigns each tile longer than
+// seg.length, unless whole_pays, its ceil(length / seg.length) checkpoint
 // slots, in tile order, into seg.index[0 .. tiles) (-1: not split, or past
 // the capacity, which the host sizes so that it is never reached).
 __global__ __launch_bounds__(kOrderBlock) void tile_order_kernel(const int* __restrict__ cost,
                                                                  const int2* __restrict__ ranges,
                                                                  int tiles,
                                                                  int* __restrict__ order,
-                                                                 Segments seg) {
+                                                                 bool neural, Segments seg) {
   __shared__ int count[kOrderBuckets];
   __shared__ int next[kOrderBuckets];
   __shared__ int scan[kOrderBlock];
   if (seg.length > 0) {
+    int longest_whole = seg.length;
+    if (tiles > kSplitAllTiles) {
+      int own = 0, longest = 0;
+      for (int t = threadIdx.x; t < tiles; t += kOrderBlock) {
+        const int length = ranges[t].y - ranges[t].x;
+        own += length > seg.length ? segment_count(length, seg.length) : 0;
+        longest = max(longest, length);
+      }
+      if (threadIdx.x == 0) next[0] = 0;
+      int segments;
+      block_inclusive_sum(own, scan, &segments);
+      longest = wave_max(longest);
+      if (lane_id() == 0) atomicMax(&next[0], longest);
+      __syncthreads();
+      if (whole_pays(neural, next[0], segments)) longest_whole = INT_MAX;
+      __syncthreads();
+    }
     int carry = 0;
     for (int first = 0; first < tiles; first += kOrderBlock) {
       const int t = first + threadIdx.x;
-      const int k = t < tiles ? segment_count(ranges[t].y - ranges[t].x, seg.length) : 1;
-      const int slots = k > 1 ? k : 0;
+      const int length = t < tiles ? ranges[t].y - ranges[t].x : 0;
+      const int slots = length > longest_whole ? segment_count(length, seg.length) : 0;
       int chunk;
       const int base = carry + block_inclusive_sum(slots, scan, &chunk) - slots;
       if (t < tiles) seg.index[t] = (slots > 0 && base + slots <= seg.capacity) ? base : -1;
@@ -1017,9 +1056,7 @@ __global__ __launch_bounds__(kOrderBlock) void tile_order_kernel(const int* __re
     }
     for (int i = total + threadIdx.x; i < tiles + seg.capacity; i += kOrderBlock)
       seg.work[i] = make_int2(-1, 0);
-    __syncthreads();
-    for (int b = threadIdx.x; b < kOrderBuckets; b += kOrderBlock) count[b] = 0;
-    __syncthreads();
+    return;
   }
   for (int b = threadIdx.x; b < kOrderBuckets; b += kOrderBlock) count[b] = 0;
   __syncthreads();
@@ -1362,8 +1399,11 @@ static_assert(kCheckpointFloats >= kSegmentResults, "a slot holds a segment's re
 // replay list, and mergeSegments completes the tile).
 // Replay: also write the tile's replay list (replay + range start, see
 // append_replay) and its length (replay_counts[tile]).
+// The split launches are bound to a wave per SIMD less: with one more the
+// classic ones spill up to 14 registers, 640x480 of 30k surfels 104 against 98
+// us (tiles walked whole).
 template <bool Neural, bool Replay, bool Split>
-__global__ __launch_bounds__(kTilePixels, Neural ? (Split ? 4 : 5) : 6) void renderForward(
+__global__ __launch_bounds__(kTilePixels, (Neural ? 5 : 6) - (Split ? 1 : 0)) void renderForward(
     int width, int height, int tw, int th, const float* __restrict__ geometry,
     const float* __restrict__ appearance, const float* __restrict__ opacities,
     const int64_t* __restrict__ primitive_ids, const float* __restrict__ backgrounds,
@@ -2979,7 +3019,8 @@ int render_forward(int32_t neural, const float* geometry, const float* appearanc
     else run(tile_probe_kernel<false>);
     GS_LAUNCHED("tile_probe_kernel");
   }
-  tile_order_kernel<<<1, kOrderBlock, 0, s>>>(probed ? probe : nullptr, r, tiles, order, seg);
+  tile_order_kernel<<<1, kOrderBlock, 0, s>>>(probed ? probe : nullptr, r, tiles, order,
+                                              neural != 0, seg);
   GS_LAUNCHED("tile_order_kernel");
   int2* lists = reinterpret_cast<int2*>(replay);
   const unsigned blocks = unsigned(seg.length ? tiles + seg.capacity : tiles);
@@ -3192,7 +3233,7 @@ int gs_render_backward(int32_t neural, const float* geometry, const float* appea
       GS_LAUNCHED("tile_last_kernel");
     }
     tile_order_kernel<<<1, kOrderBlock, 0, s>>>(replay ? replay_counts : w.tile_last, r, tiles,
-                                                w.order, seg);
+                                                w.order, neural != 0, seg);
     GS_LAUNCHED("tile_order_kernel");
   }
   const int2* lists = reinterpret_cast<const int2*>(replay);

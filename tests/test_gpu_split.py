@@ -11,12 +11,13 @@ each from a checkpoint the merge wrote.
   longer than the segment length, non-decreasing replay lengths ending at
   the tile's replay count, and a last checkpoint equal to the saved state.
 * Gradients of a scene whose tiles are split match the float64 oracle.
+* Beyond 256 tiles the lists decide whether the long tiles are split.
 """
 
 import pytest
 import torch
 
-from diff_gabor_splatting_amd import _native
+from diff_gabor_splatting_amd import _native, fixed_capacity
 from oracle import render as oracle_render
 from scenes import (assert_gradients_close, fp32_conditioned, maps_from_result,
                     oracle_reference, random_scene)
@@ -214,6 +215,56 @@ def test_slots_past_capacity_leave_later_tiles_unsplit(method, monkeypatch):
     assert torch.equal(contributors, seen[-1][4])
     torch.testing.assert_close(capped_maps, plain_maps, atol=2e-6, rtol=2e-5)
     for name, a, b in zip(values, capped_grads, plain_grads):
+        scale = float(b.abs().max())
+        err = float((a - b).abs().max())
+        assert err <= 1e-3 * scale + 1e-12, f"{name}: max error {err:.3e}, scale {scale:.3e}"
+
+
+def walked_whole(method, tiles, longest, segments):
+    """The compositor's rule (whole_pays in composite.hip)."""
+    if tiles <= 256:
+        return False
+    return longest <= (segments // 7 - 100 if method == "neural" else max(segments // 5, 170))
+
+
+@pytest.mark.parametrize("method", ["classic", "neural"])
+@pytest.mark.parametrize("cameras, width, height, spread, whole", [
+    (5, 250, 255, 1.0, True),    # even lists, 1,280 tiles
+    (5, 250, 255, 0.15, False),  # a few long lists
+    (1, 256, 256, 1.0, False),   # 256 tiles are split in any case
+    (1, 272, 256, 0.15, False),
+])
+def test_whole_or_split(method, cameras, width, height, spread, whole, monkeypatch):
+    """Beyond 256 tiles the lists decide on the device whether the long tiles
+    are split, all or none: the decision is the rule's, the same in a
+    fixed-capacity render (same bits), and the results are the unsplit
+    render's to float32 rounding, as for every split."""
+    raw = random_scene(method, scenes=1, cameras=cameras, n=1500, width=width, height=height,
+                       seed=3, focal=330.0)
+    raw["means"][..., :2] *= spread
+    values = {k: v.to(DEVICE).requires_grad_() for k, v in raw.items()}
+    weights = torch.randn((1, cameras, height, width, 9),
+                          generator=torch.Generator().manual_seed(8)).to(DEVICE)
+    print(f"whole or split: {method} {cameras} x {width}x{height} spread {spread}", flush=True)
+    seen = spy_forward(monkeypatch)
+    maps, grads = run(method, values, weights, width, height)
+    _, _, ranges, _, contributors, (_, _, (length, _, index)) = seen[-1]
+    tiles = ranges.shape[0]
+    lengths = (ranges[:, 1] - ranges[:, 0]).long()
+    segments = int(((lengths + length - 1) // length)[lengths > length].sum())
+    print(f"longest {int(lengths.max())}, {segments} segments of {tiles} tiles", flush=True)
+    assert walked_whole(method, tiles, int(lengths.max()), segments) == whole
+    assert torch.equal(index[:tiles] >= 0, (lengths > length) & (not whole))
+    capacity = int(lengths.sum()) + 777
+    with torch.no_grad(), fixed_capacity(capacity):
+        bounded = maps_from_result(renderer(method)(**values, width=width, height=height))
+    assert torch.equal(bounded, maps)
+    monkeypatch.setattr(_native, "SPLIT_MAX_TILES", 0)
+    plain_maps, plain_grads = run(method, values, weights, width, height)
+    assert seen[-1][5][2] is None
+    assert torch.equal(contributors, seen[-1][4])
+    torch.testing.assert_close(maps, plain_maps, atol=2e-6, rtol=2e-5)
+    for name, a, b in zip(values, grads, plain_grads):
         scale = float(b.abs().max())
         err = float((a - b).abs().max())
         assert err <= 1e-3 * scale + 1e-12, f"{name}: max error {err:.3e}, scale {scale:.3e}"
