@@ -23,6 +23,7 @@
 // or tile-block ids.
 #include "sort.hpp"
 
+#include <algorithm>
 #include <type_traits>
 
 #include "scan.hpp"
@@ -32,12 +33,20 @@ namespace {
 
 constexpr int kSortBlock = 256;
 constexpr int kSortWaves = kSortBlock / 64;
-// Keys per thread: 16 (4096-key spans), or 8 for sorts of up to
-// kShortSort keys, which then spread over twice as many workgroups - a
-// 1M-key sort otherwise leaves a 256-CU device with one span per CU.
+// Keys per thread: 16 (4096-key spans), or fewer for shorter sorts, which
+// then spread over more workgroups: a 1M-key sort of 16 leaves a 256-CU
+// device with one span per CU, and below that the passes take as long as one
+// span's serial ranking (a ballot per digit bit and key). Against that stand
+// each span's counters and prefix sums. 27 bits with values, three passes,
+// at 8, 4 and 2 keys per thread: 20k keys 42.2, 34.4, 31.1 us, 80k 44.6, 37.1,
+// 34.8, 160k 46.4, 40.8, 44.1, 300k 50.3, 50.4, 56.8.
+constexpr int64_t kTinySort = int64_t(3) << 15;
+constexpr int64_t kSmallSort = int64_t(1) << 18;
 constexpr int64_t kShortSort = int64_t(1) << 22;
 __host__ __device__ constexpr int span_keys(int items) { return kSortBlock * items; }
-int sort_items(int64_t m) { return m <= kShortSort ? 8 : 16; }
+int sort_items(int64_t m) {
+  return m <= kTinySort ? 2 : m <= kSmallSort ? 4 : m <= kShortSort ? 8 : 16;
+}
 constexpr int kDigitBits = 8;
 constexpr int kBins = 1 << kDigitBits;
 // Multi-workgroup passes of 32-bit keys may take digits of up to
@@ -430,7 +439,13 @@ struct SortWorkspace {
 };
 
 SortWorkspace layout(void* base, int64_t m, int key_bytes) {
-  const int64_t spans = ceil_div(m, span_keys(sort_items(m)));
+  // The spans of the longest sorts of each kind up to m keys, so that scratch
+  // for m keys also holds any shorter sort.
+  int64_t spans = 0;
+  for (const int64_t most : {kTinySort, kSmallSort, kShortSort, m}) {
+    const int64_t n = std::min(m, most);
+    spans = std::max(spans, ceil_div(n, span_keys(sort_items(n))));
+  }
   const int64_t count_items = int64_t(kWideBins) * spans;
   SortWorkspace w;
   size_t offset = 0;
@@ -527,23 +542,25 @@ int radix_sort(const Key* keys_in, Key* keys_out, const int* values_in, int* val
         radix_downsweep_kernel<Key, I, false, B><<<unsigned(spans), kSortBlock, 0, s>>>(
             src_k, src_v, dst_k, dst_v, m, live, shift, bits, w.counts, w.totals, spans);
     };
-    auto run = [&](auto bins_tag) {
-      using Items8 = std::integral_constant<int, 8>;
-      using Items16 = std::integral_constant<int, 16>;
+    auto run = [&](auto items_tag, auto bins_tag) {
       constexpr int B = decltype(bins_tag)::value;
-      if (items == 8) upsweep(Items8{}, bins_tag);
-      else upsweep(Items16{}, bins_tag);
+      upsweep(items_tag, bins_tag);
       GS_LAUNCHED("radix_upsweep_kernel");
       scan_rows_kernel<<<B, kSortBlock, 0, s>>>(w.counts, spans, w.totals, m, live,
                                                 span_keys(items));
       GS_LAUNCHED("scan_rows_kernel");
-      if (items == 8) downsweep(Items8{}, bins_tag);
-      else downsweep(Items16{}, bins_tag);
+      downsweep(items_tag, bins_tag);
       GS_LAUNCHED("radix_downsweep_kernel");
       return GS_OK;
     };
-    const int status = bins == kBins ? run(std::integral_constant<int, kBins>{})
-                                     : run(std::integral_constant<int, kWideBins>{});
+    auto by_items = [&](auto bins_tag) {
+      if (items == 2) return run(std::integral_constant<int, 2>{}, bins_tag);
+      if (items == 4) return run(std::integral_constant<int, 4>{}, bins_tag);
+      if (items == 8) return run(std::integral_constant<int, 8>{}, bins_tag);
+      return run(std::integral_constant<int, 16>{}, bins_tag);
+    };
+    const int status = bins == kBins ? by_items(std::integral_constant<int, kBins>{})
+                                     : by_items(std::integral_constant<int, kWideBins>{});
     if (status != GS_OK) return status;
     src_k = dst_k;
     src_v = dst_v;

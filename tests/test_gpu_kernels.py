@@ -82,6 +82,23 @@ def test_local_sort_items(native, m, bits, with_values):
         np.testing.assert_array_equal(sv.cpu().numpy(), values[order])
 
 
+@pytest.mark.parametrize("m", [8193, 8704, 98_303, 98_304, 98_305, 262_144, 262_145])
+def test_sort_items_edges(native, m):
+    """Digit passes at the edges of their keys per thread (2, 4 and 8): 27 bits
+    in three 9-bit passes, with values. Scratch for m keys holds any shorter
+    sort."""
+    rng = np.random.default_rng(m)
+    keys = rng.integers(0, 2**27, m, dtype=np.uint64).astype(np.uint32)
+    keys[m // 2:] = keys[: m - m // 2]  # ties across spans
+    sk, sv = native.sort_pairs32(torch.from_numpy(keys.view(np.int32)).to(DEVICE),
+                                 torch.arange(m, dtype=torch.int32, device=DEVICE), 0, 27)
+    order = np.argsort(keys, kind="stable")
+    np.testing.assert_array_equal(sk.cpu().numpy().view(np.uint32), keys[order])
+    np.testing.assert_array_equal(sv.cpu().numpy(), order)
+    size = native.lib.gs_sort32_workspace_size
+    assert size(m - 1) <= size(m) <= size(m + 1) <= size(2 * m)
+
+
 @pytest.mark.parametrize("m", [1, 5, 4095, 4096, 4097, 8192, 8193, 100_003, 2_000_000])
 @pytest.mark.parametrize("bits", [(0, 64), (0, 45), (32, 45), (3, 17)])
 def test_sort_is_stable_radix_order(native, m, bits):
