@@ -268,3 +268,26 @@ def test_whole_or_split(method, cameras, width, height, spread, whole, monkeypat
         scale = float(b.abs().max())
         err = float((a - b).abs().max())
         assert err <= 1e-3 * scale + 1e-12, f"{name}: max error {err:.3e}, scale {scale:.3e}"
+
+
+@pytest.mark.parametrize("length", [64, 192])
+@pytest.mark.parametrize("n", [300, 5600])
+def test_replay_blocks_are_packed(length, n, monkeypatch):
+    """The merge packs the segments' replay blocks into one list, 64 segments
+    and four 64-entry chunks at a time: the same entries, in order, as an
+    unsplit render's (lists of up to 71 segments; segments of one and of three
+    chunks)."""
+    width, height = 24, 20
+    values = heavy_scene("classic", 0.02, n=n, width=width, height=height)
+    seen = spy_forward(monkeypatch)
+    monkeypatch.setattr(_native, "SPLIT_LENGTH", length)
+    renderer("classic")(**values, width=width, height=height)
+    monkeypatch.setattr(_native, "SPLIT_MAX_TILES", 0)
+    renderer("classic")(**values, width=width, height=height)
+    (_, _, ranges, _, _, (lists, counts, segments)) = seen[0]
+    (_, _, _, _, _, (plain_lists, plain_counts, none)) = seen[1]
+    assert none is None and int((segments[2][:ranges.shape[0]] >= 0).sum()) > 0
+    print(f"lists of up to {int((ranges[:, 1] - ranges[:, 0]).max())} records", flush=True)
+    assert torch.equal(counts, plain_counts)
+    for (first, _), count in zip(ranges.tolist(), counts.tolist()):
+        assert torch.equal(lists[first:first + count], plain_lists[first:first + count])
