@@ -2250,24 +2250,26 @@ __global__ __launch_bounds__(kTilePixels, (backward_occupancy<Neural, Replay>())
 //    chunks stays in LDS;
 //  * per step a lane reads its pixel's 16 constants (four 16-byte LDS reads,
 //    one address per 16-lane row).
-// The waves of a workgroup share nothing but the tile, so there is no barrier
-// after the prologue and no batch: each wave ends when its own list does.
+// A record's sums over the tile's four quadrants meet in LDS, a window of
+// entries at a time (kWindow), where one thread per record turns them into its
+// gradients: one global atomic per (tile, record, parameter), as in the walk with
+// a pixel per lane. Atomics on one cache line follow each other at about 27 ns,
+// so with one per quadrant 16 surfels that fill 1920x1080 took 1,045 us (now
+// 325, a pixel per lane 350), and a record's gradient rounded four times as often.
 //
 // It is bound by VALU issue: about 170 instructions per step of 64 samples and
-// 300 per chunk around the steps, against 253 per record and wave with a pixel
-// per lane. Measured, kernel alone: 1M surfels at 1920x1080, all maps, 1.167 ->
-// 0.986 ms; 100k at 1024x768, rgb, alpha and depth, 0.448 -> 0.388 ms; 32 views
-// at 512x512 4.74 -> 4.01 ms. Three waves per SIMD without spills are 2% faster
-// than four with 14 spilled registers. The neural adjoint has 57 sums and 55
-// record constants, which leave two waves per SIMD, and stays with a pixel per
-// lane (0.684 ms against 0.714 on 100k surfels at 800x800). An f32 MFMA per four
+// 150 per chunk around the steps, against 253 per record and wave with a pixel
+// per lane. Measured, kernel alone: 1M surfels at 1920x1080, all maps, 1.145 ->
+// 0.935 ms; 100k at 1024x768, rgb, alpha and depth, 0.446 -> 0.330 ms; 32 views
+// at 512x512 4.63 -> 3.73 ms. The neural adjoint has 54 sums and 55 record
+// constants, which leave two waves per SIMD, and stays with a pixel per lane
+// (0.684 ms against 0.714 on 100k surfels at 800x800). An f32 MFMA per four
 // pixels in place of the products with per-pixel values (20 multiply-adds for 6
 // MFMAs) is slower (1.23 ms): each takes its 32 cycles of the SIMD.
 namespace by_record {
 
-constexpr int kChunk = 16;              // records per chunk: one DPP row
-constexpr int kGroups = 64 / 4;         // pixel steps per chunk
-constexpr int kQueue = 128;             // ring of filtered replay entries per wave
+constexpr int kChunk = 16;       // records per chunk: one DPP row
+constexpr int kGroups = 64 / 4;  // pixel steps per chunk
 
 // A pixel's constants in LDS: position, last contributor (int bits), the
 // term of dL/dalpha that all records share, map gradients (rgb, depth,
@@ -2370,6 +2372,41 @@ __device__ __forceinline__ void wave_lds_fence() {
   __builtin_amdgcn_wave_barrier();
 }
 
+// to[j] += v[j] in LDS for j < count, atomically against the workgroup's other
+// waves, with integer exchanges: a float LDS atomic takes about 1.5 cycles per
+// lane, which made the whole kernel 30% slower (1M surfels at 1920x1080 1.32
+// against 0.96 ms). A cell's content is taken (0 left in it), added to and put
+// back; if another wave put its sum in between, that sum comes back and is added
+// again. Each time some wave finds nothing to take back, so of the four that may
+// meet at a cell one at least is done with every turn.
+template <int N>
+__device__ __forceinline__ void shared_add(float* to, float (&v)[N], int count) {
+  auto exchange = [](float* cell, float value) {
+    return __uint_as_float(__hip_atomic_exchange(reinterpret_cast<uint32_t*>(cell),
+                                                 __float_as_uint(value), __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_WORKGROUP));
+  };
+#pragma unroll
+  for (int j = 0; j < N; ++j)
+    if (j < count) v[j] += exchange(to + j, 0.f);
+  uint32_t back = 0;
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    v[j] = j < count ? exchange(to + j, v[j]) : 0.f;
+    back |= __float_as_uint(v[j]);
+  }
+  while (back) {
+    back = 0;
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+      if (__float_as_uint(v[j]) != 0u) {
+        v[j] += exchange(to + j, 0.f);
+        v[j] = exchange(to + j, v[j]);
+        back |= __float_as_uint(v[j]);
+      }
+  }
+}
+
 // One record's constants in a lane's registers.
 struct Record {
   float row[15];  // what sample_surface reads: T 0-8, centre 9-10, normal 11-13, opacity 14
@@ -2382,10 +2419,10 @@ struct Record {
 
 // Loads record `id` (appearance row and opacity of primitive `prim`) and
 // derives its constants; lanes without a record (present = false) take the
-// opacity 0, which no pixel accepts. (centre_x, centre_y) of the quadrant bound
-// the record's centre to kCentreReach pixels around it: further out no pixel of
-// the quadrant passes by rho2 (accepted samples have rho <= 2 ln(255 o) < 190 for
-// any float opacity, rho2 > 7000), so no decision changes, while the centre of a
+// opacity 0, which no pixel accepts. (centre_x, centre_y) of the tile bound the
+// record's centre to kCentreReach pixels around it: further out no pixel of the
+// tile passes by rho2 (accepted samples have rho <= 2 ln(255 o) < 190 for any
+// float opacity, rho2 > 6000), so no decision changes, while the centre of a
 // surfel that crosses the camera plane can lie anywhere and would cost the moment
 // sums X and Y their precision. colour_sums (c1 + c2) is what only
 // record_gradients needs.
@@ -2627,22 +2664,37 @@ __device__ __forceinline__ void record_gradients(const Record& rec, const float*
   to[kClassic] = v[S::OPACITY];
 }
 
-constexpr int kGeometryOut = 14;                        // geometry columns written
+constexpr int kGeometryOut = 14;                       // geometry columns written
 constexpr int kOutputs = kGeometryOut + kClassic + 1;  // per record
 constexpr int kSumPitch = 37;  // a record's sums, then its outputs in their place
 static_assert(kSumPitch >= kOutputs && kSumPitch >= Sums<kAllMaps>::COUNT, "a record's LDS row");
 
+// Replay entries whose sums a tile holds in LDS at once: as many as let the
+// workgroups that the registers allow stay on a CU (three with all maps, in 50 KB
+// each, else four, in 40 KB). Of a longer list each window ends with the waves
+// waiting for each other and, on average, half a chunk per quadrant: all maps of
+// 1M surfels at 1920x1080 (lists of 128 on average, up to 368) 930 us with 192,
+// 956 with 128, 977 with 112; rgb, alpha and depth of 100k at 1024x768 318 us
+// with 128, 326 with 192.
+template <int Maps>
+constexpr int kWindow = Maps == kAllMaps ? 192 : 128;
+
+template <int Maps>
 struct Wave {
   float pixels[64 * ReplayPixel::FLOATS];
   float2 state[64];
-  // The chunk's sums; during the walk, where lanes without a state to keep
-  // write theirs.
-  float sums[kChunk * kSumPitch];
-  float colour_sums[kChunk * 3];
-  uint64_t rows[kChunk][2];  // the gradient rows of the chunk's records
-  int ids[kQueue];
-  uint32_t prims[kQueue];
-  int positions[kQueue];
+  uint8_t taken[kWindow<Maps>];  // the window's entries that the quadrant took
+};
+
+// A window of the tile's replay list: its entries and their sums over the tile.
+template <int Maps>
+struct Window {
+  static_assert(kWindow<Maps> <= kTilePixels && kWindow<Maps> <= 256,
+                "a thread and a uint8_t index per entry");
+  int ids[kWindow<Maps>];
+  uint32_t prims[kWindow<Maps>];
+  int words[kWindow<Maps>];  // list position and quadrant bits (append_replay)
+  float sums[kWindow<Maps> * kSumPitch];
 };
 
 // The replay walk's backward compositor: one workgroup per tile, or per
@@ -2661,7 +2713,9 @@ __global__ __launch_bounds__(kTilePixels, 3) void renderBackward(
     const int2* __restrict__ segments, Segments seg) {
   using S = Sums<Maps>;
   using P = ReplayPixel;
-  __shared__ __align__(16) Wave waves[kTilePixels / 64];
+  __shared__ __align__(16) Wave<Maps> waves[kTilePixels / 64];
+  __shared__ Window<Maps> window;
+  __shared__ float2 aside[64];  // where lanes without a pixel state to keep write theirs
   __shared__ float bg_acc[3];
   const int lane = lane_id();
   // (tile, segment) of this workgroup; past the segment count: nothing.
@@ -2669,7 +2723,7 @@ __global__ __launch_bounds__(kTilePixels, 3) void renderBackward(
   if (piece.x < 0) return;
   const int tile = piece.x;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  Wave& lds = waves[wave];
+  Wave<Maps>& lds = waves[wave];
 #ifdef GS_DIAGNOSTICS
   const long long diag_begin = wall_clock64();
   __shared__ unsigned int diag_lanes[65];
@@ -2768,57 +2822,37 @@ __global__ __launch_bounds__(kTilePixels, 3) void renderBackward(
   auto uniform = [](float v) {
     return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
   };
-  const float centre_x = uniform(float(tp.px - (lane & 7)) + 3.5f);
-  const float centre_y = uniform(float(tp.py - (lane >> 3)) + 3.5f);
+  // The tile's centre.
+  const float centre_x = uniform(float(tp.px - (lane & 7) - 8 * (wave & 1)) + 7.5f);
+  const float centre_y = uniform(float(tp.py - (lane >> 3) - 8 * (wave >> 1)) + 7.5f);
   const int quadrant = kReplayPositionBits + wave;
   // Lane 15 of a row keeps its pixel's state, the others write theirs aside.
-  float2* const aside = reinterpret_cast<float2*>(lds.sums);
   float2* const state_row = (slot == kChunk - 1 ? lds.state : aside) + row;
-  static_assert(kChunk * kSumPitch >= 2 * 64, "the sums hold a quadrant's states");
 
-  auto walk_chunks = [&](auto masked) {
+  // The wave's part of a window of n entries: those its quadrant took.
+  auto walk_window = [&](auto masked, int n) {
     constexpr bool kMasked = decltype(masked)::value;
-    int head = 0, tail = 0;  // ring positions: queued entries are [head, tail)
-    int next = block_last;   // entries [block_first, next) are still to be read
-    // Entry read ahead of the wave's next 64.
-    int2 ahead = make_int2(0, 0);
-    if (next - 1 - lane >= block_first) ahead = replay[range.x + next - 1 - lane];
-    while (true) {
-      // Queue the quadrant's entries until a chunk is full or none are left.
-      while (tail - head < kChunk && next > block_first) {
-        const bool keep = next - 1 - lane >= block_first && ((uint32_t(ahead.y) >> quadrant) & 1u);
-        const uint64_t kept = __ballot(keep);
-        if (keep) {
-          const int before = int(__builtin_amdgcn_mbcnt_hi(
-              uint32_t(kept >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(kept), 0u)));
-          const int at = (tail + before) & (kQueue - 1);
-          lds.ids[at] = ahead.x;
-          lds.positions[at] = (ahead.y & kReplayPositionMask) + 1;
-          lds.prims[at] = uint32_t(primitive_ids[ahead.x]);
-        }
-        tail += __popcll(kept);
-        next -= 64;
-        if (next - 1 - lane >= block_first) ahead = replay[range.x + next - 1 - lane];
-      }
-      const int n = min(kChunk, tail - head);
-      if (n <= 0) break;
-      wave_lds_fence();
-      const int at = (head + min(slot, n - 1)) & (kQueue - 1);
-      const int id = lds.ids[at];
-      const uint32_t prim = lds.prims[at];
-      head += n;
+    int count = 0;
+    for (int first = 0; first < n; first += 64) {
+      const int entry = n - 1 - first - lane;
+      const bool keep = entry >= 0 && ((uint32_t(window.words[max(entry, 0)]) >> quadrant) & 1u);
+      const uint64_t kept = __ballot(keep);
+      const int before = int(__builtin_amdgcn_mbcnt_hi(
+          uint32_t(kept >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(kept), 0u)));
+      if (keep) lds.taken[count + before] = uint8_t(entry);
+      count += __popcll(kept);
+    }
+    wave_lds_fence();
+    for (int done = 0; done < count; done += kChunk) {
+      const int in_chunk = min(kChunk, count - done);
+      const int entry = lds.taken[done + min(slot, in_chunk - 1)];
+      const int id = window.ids[entry];
+      const uint32_t prim = window.prims[entry];
+      const int position = (window.words[entry] & kReplayPositionMask) + 1;
       Record rec;
       float colour_sums[3];
-      load_record(rec, colour_sums, slot < n, id, prim, lds.positions[at], centre_x, centre_y,
-                          geometry, appearance, opacities);
-      auto address = [](const float* t) { return reinterpret_cast<uint64_t>(t); };
-      if (row == 0) {
-#pragma unroll
-        for (int c = 0; c < 3; ++c) lds.colour_sums[slot * 3 + c] = colour_sums[c];
-        lds.rows[slot][0] = address(grad_geometry) + uint64_t(int64_t(id) * kGeometry) * 4;
-        lds.rows[slot][1] =
-            address(grad_appearance) + uint64_t(prim) * (kClassic * 4) - kGeometryOut * 4;
-      }
+      load_record(rec, colour_sums, slot < in_chunk, id, prim, position, centre_x, centre_y,
+                  geometry, appearance, opacities);
       float sum[S::COUNT];
 #pragma unroll
       for (int i = 0; i < S::COUNT; ++i) sum[i] = 0.f;
@@ -2849,7 +2883,7 @@ __global__ __launch_bounds__(kTilePixels, 3) void renderBackward(
 #ifdef GS_DIAGNOSTICS
       took |= __shfl_xor(took, 16, 64);
       took |= __shfl_xor(took, 32, 64);
-      for (int j = 0; j < n; ++j) {
+      for (int j = 0; j < in_chunk; ++j) {
         const uint64_t taking = __shfl(took, j, 64);
         if (lane == 0 && taking) atomicAdd(&diag_lanes[__popcll(taking)], 1u);
         if (taking) packing.add(taking);
@@ -2857,48 +2891,63 @@ __global__ __launch_bounds__(kTilePixels, 3) void renderBackward(
       packing.flush(diag_packing);
 #endif
       wave_lds_fence();
-      // The record's sums over the four pixel rows, then its gradients.
-      {
-        using R = RowSums<S::COUNT>;
-        float part[R::ROW];
-        R::reduce(sum, part, lane);
-        float* to = lds.sums + slot * kSumPitch + R::first(row);
-        const int count = R::count(row);
-#pragma unroll
-        for (int j = 0; j < R::ROW; ++j)
-          if (j < count) to[j] = part[j];
-      }
-      wave_lds_fence();
-      if (lane < n) {
-        float* out = lds.sums + lane * kSumPitch;
-        record_gradients<Maps>(rec, lds.colour_sums + lane * 3, out);
-      }
-      wave_lds_fence();
-      // One global atomic per nonzero output; consecutive lanes take
-      // consecutive columns of a record, so that a wave's atomics fall on a few
-      // cache lines.
-      // Half a wave per record: columns 0..13 geometry, 14..31 appearance.
-      static_assert(kOutputs == 33, "32 columns and the opacity");
-      const int p = lane & 31, half = lane >> 5;
-      const uint64_t* base = &lds.rows[half][p >= kGeometryOut];
-      const float* value = lds.sums + half * kSumPitch + p;
-#pragma unroll
-      for (int j = 0; j < kChunk; j += 2) {
-        const float v = value[j * kSumPitch];
-        if (j + half < n && v != 0.f) global_add(base[2 * j] + p * 4, v);
-      }
-      if (lane < n) {
-        const float v = lds.sums[lane * kSumPitch + 32];
-        if (v != 0.f) global_add(address(grad_opacities + prim), v);
-      }
-      // The ring's consumed slots and the sums may be overwritten from here on.
-      wave_lds_fence();
+      // The record's sums over the four pixel rows, into the tile's.
+      using R = RowSums<S::COUNT>;
+      float part[R::ROW];
+      R::reduce(sum, part, lane);
+      float* to = window.sums + entry * kSumPitch + R::first(row);
+      if (slot < in_chunk) shared_add(to, part, R::count(row));
     }
   };
-  if (finite_pixels)
-    walk_chunks(std::false_type{});
-  else
-    walk_chunks(std::true_type{});
+
+  // Equal windows, from the last to the first.
+  const int total = block_last - block_first;
+  const int windows = (total + kWindow<Maps> - 1) / kWindow<Maps>;
+  const int size = windows ? (total + windows - 1) / windows : 0;
+  for (int last = total; last > 0; last -= size) {
+    const int n = min(size, last);
+    if (int(threadIdx.x) < n) {
+      const int2 e = replay[range.x + block_first + last - n + int(threadIdx.x)];
+      window.ids[threadIdx.x] = e.x;
+      window.words[threadIdx.x] = e.y;
+      window.prims[threadIdx.x] = uint32_t(primitive_ids[e.x]);
+    }
+    for (int i = threadIdx.x; i < n * kSumPitch; i += kTilePixels) window.sums[i] = 0.f;
+    __syncthreads();
+    if (finite_pixels)
+      walk_window(std::false_type{}, n);
+    else
+      walk_window(std::true_type{}, n);
+    __syncthreads();
+    // One thread per record turns its sums into its gradients, in place.
+    if (int(threadIdx.x) < n) {
+      Record rec;
+      float colour_sums[3];
+      load_record(rec, colour_sums, true, window.ids[threadIdx.x], window.prims[threadIdx.x], 0,
+                  centre_x, centre_y, geometry, appearance, opacities);
+      record_gradients<Maps>(rec, colour_sums, window.sums + threadIdx.x * kSumPitch);
+    }
+    __syncthreads();
+    // One global atomic per nonzero output; consecutive lanes take consecutive
+    // columns of a record, so that a wave's atomics fall on a few cache lines.
+    // Half a wave per record: columns 0..13 geometry, 14..31 appearance.
+    static_assert(kOutputs == 33, "32 columns and the opacity");
+    const int p = threadIdx.x & 31;
+    auto address = [](const float* t) { return reinterpret_cast<uint64_t>(t); };
+    for (int j = threadIdx.x >> 5; j < n; j += kTilePixels / 32) {
+      const float v = window.sums[j * kSumPitch + p];
+      const uint64_t to = p < kGeometryOut
+                              ? address(grad_geometry) + uint64_t(int64_t(window.ids[j]) * kGeometry) * 4
+                              : address(grad_appearance) +
+                                    uint64_t(window.prims[j]) * (kClassic * 4) - kGeometryOut * 4;
+      if (v != 0.f) global_add(to + p * 4, v);
+    }
+    if (int(threadIdx.x) < n) {
+      const float v = window.sums[threadIdx.x * kSumPitch + 32];
+      if (v != 0.f) global_add(address(grad_opacities + window.prims[threadIdx.x]), v);
+    }
+    __syncthreads();  // before the next window overwrites this one
+  }
 #ifdef GS_DIAGNOSTICS
   __syncthreads();
   if (gs_diagnostics.lanes && threadIdx.x < 65 && diag_lanes[threadIdx.x] != 0u)

@@ -1,10 +1,10 @@
 """The classic replay backward, whose lanes are 16 records x 4 pixels.
 
-Its chunks of 16 records, its queue of filtered entries (refilled 64 at a
-time) and its three variants by the gradient groups present are checked on
-stacks of surfels that every pixel takes, at lengths around those sizes,
-against the full-list walk, which keeps one pixel per lane, sums across the
-wave and derives every row of T per pixel.
+Its chunks of 16 records, its windows of 128 or 192 entries and its three
+variants by the gradient groups present are checked on stacks of surfels that
+every pixel takes, at lengths around those sizes, against the full-list walk,
+which keeps one pixel per lane, sums across the wave and derives every row of T
+per pixel.
 
 Both take the same records with the same per-sample float32 values; they
 differ in the order of the sums over at most 256 pixels and n records, so a
@@ -15,6 +15,8 @@ goes with rgb: its own dL/dw, m^2 A + m2 - 2 m m1, keeps (dm / m)^2 ~ 6e-4 of
 its terms and dL/dalpha is a difference of such values, so alone it is known
 to 1e-4 at best on either side.
 """
+
+import math
 
 import pytest
 import torch
@@ -53,20 +55,24 @@ def stack(n, seed):
     return {k: v.contiguous().to(DEVICE) for k, v in values.items()}
 
 
-def gradients(values, gradient_groups, non_finite=False):
+GROUPS = {"rgb": (1, 0, 0, 0, 0), "rgb+alpha": (1, 1, 0, 0, 0), "depth": (1, 1, 1, 0, 0),
+          "normals": (0, 0, 0, 1, 0), "rgb+distortion": (1, 0, 0, 0, 1), "all": (1, 1, 1, 1, 1)}
+
+
+def gradients(values, gradient_groups, non_finite=False, width=WIDTH, height=HEIGHT):
     """(by record, full list) gradients of one render."""
     from diff_gabor_splatting_amd import _native
 
-    args = compositor_inputs(renderer(False), values, dict(width=WIDTH, height=HEIGHT))
+    args = compositor_inputs(renderer(False), values, dict(width=width, height=height))
     maps, points, ranges, state, contributors, replay = _native.rasterize_forward(
         *args, replay=True)
     saved = (*args[:4], args[6], points, ranges, state, contributors)
     g = torch.Generator().manual_seed(7)
-    groups = [torch.randn(1, HEIGHT, WIDTH, k, generator=g).to(DEVICE) if on else None
+    groups = [torch.randn(1, height, width, k, generator=g).to(DEVICE) if on else None
               for k, on in zip((3, 1, 1, 3, 1), gradient_groups)]
     if non_finite:
         groups[0][0, 2, 3, 1] = float("inf")
-    return [_native.rasterize_backward(*saved, groups, WIDTH, HEIGHT, False, *args[10:12],
+    return [_native.rasterize_backward(*saved, groups, width, height, False, *args[10:12],
                                        replay=lists) for lists in (replay, None)]
 
 
@@ -74,10 +80,89 @@ def gradients(values, gradient_groups, non_finite=False):
 @pytest.mark.parametrize("present", ["rgb", "rgb+alpha", "depth", "normals", "rgb+distortion",
                                      "all"])
 def test_chunks_match_the_full_walk(n, present):
-    on = {"rgb": (1, 0, 0, 0, 0), "rgb+alpha": (1, 1, 0, 0, 0), "depth": (1, 1, 1, 0, 0),
-          "normals": (0, 0, 0, 1, 0), "rgb+distortion": (1, 0, 0, 0, 1), "all": (1, 1, 1, 1, 1)}
-    for a, e in zip(*gradients(stack(n, n), on[present])):
+    for a, e in zip(*gradients(stack(n, n), GROUPS[present])):
         assert float((a - e).norm()) <= 1e-5 * float(e.norm())
+
+
+@pytest.mark.parametrize("n", [127, 128, 129, 191, 192, 193, 257, 400])
+@pytest.mark.parametrize("present", ["rgb", "depth", "all"])
+def test_windows_match_the_full_walk(n, present):
+    """Lists around the windows' edges (128 entries, with all maps 192) and of
+    several windows. The bound grows with the root of the list's length from
+    the 1e-5 at 145."""
+    values = stack(n, n)
+    values["opacities"].mul_(0.4)  # some 400 records before a pixel stops
+    for a, e in zip(*gradients(values, GROUPS[present])):
+        assert float((a - e).norm()) <= 1e-5 * max(1, n / 145) ** 0.5 * float(e.norm())
+
+
+@pytest.mark.parametrize("present", ["rgb", "depth", "all"])
+def test_centres_far_from_the_tile(present):
+    """Wide and steeply tilted surfels whose centres lie more than the 64 pixels
+    away that the moment sums' reference point is held within. There the sums
+    about that point and the rows of T about it are both of the size of the
+    affine functions k and l at the pixel (both grow with the distance), so the
+    bound stays that of the other scenes."""
+    n, width, height = 60, 640, 40
+    values = stack(n, 5)
+    g = torch.Generator().manual_seed(6)
+
+    def uniform(low, high):
+        return torch.rand(1, n, generator=g) * (high - low) + low
+
+    values["means"][..., 0] = uniform(-2.5, 2.5).to(DEVICE)
+    values["scales"][..., 0] = uniform(0.5, 4.0).to(DEVICE)
+    angle = uniform(-0.7, 0.7)  # half the rotation about y: up to 80 degrees
+    zero = torch.zeros_like(angle)
+    values["quaternions"] = torch.stack([angle.cos(), zero, angle.sin(), zero], -1).to(DEVICE)
+    values["intrinsics"] = torch.tensor(
+        [[[[300.0, 0, 320], [0, 300.0, 20], [0, 0, 1.0]]]], device=DEVICE)
+    args = compositor_inputs(renderer(False), values, dict(width=width, height=height))
+    from diff_gabor_splatting_amd import _native
+
+    _, points, ranges, _, _, (lists, counts, _) = _native.rasterize_forward(*args, replay=True)
+    far = 0
+    for tile, ((first, _), count) in enumerate(zip(ranges.tolist(), counts.tolist())):
+        centre = 16 * (tile % (width // 16)) + 7.5
+        x = args[0][lists[first:first + count, 0].long(), 9]
+        far += int(((x - centre).abs() > 64).sum())
+    print(f"{far} records of tiles with a centre more than 64 px away", flush=True)
+    assert far > 200
+    for a, e in zip(*gradients(values, GROUPS[present], width=width, height=height)):
+        assert float((a - e).norm()) <= 1e-5 * float(e.norm())
+
+
+def test_a_record_rounds_once_per_tile():
+    """A record's gradient takes one atomic addition per tile, not one per
+    quadrant: m additions of one sign round by ulp / sqrt(12) each, on average
+    2.5e-8 of the partial sum, in all 2.5e-8 sqrt(m / 3) of the total. m = 1,024
+    tiles give 4.6e-7 and 4,096 quadrants 9.2e-7; the root mean square over 48
+    sums is known to a tenth of itself, and the bound lies between."""
+    from diff_gabor_splatting_amd import _native
+
+    images, size = 16, 512
+    values = stack(1, 1)
+    values["means"] = torch.tensor([[[0.0, 0.0, 2.0]]], device=DEVICE)
+    values["quaternions"] = torch.tensor([[[1.0, 0, 0, 0]]], device=DEVICE)
+    values["scales"] = torch.full((1, 1, 2), 50.0, device=DEVICE)
+    values["view_matrices"] = torch.eye(4, device=DEVICE).repeat(1, images, 1, 1)
+    values["intrinsics"] = torch.tensor(
+        [[400.0, 0, 256], [0, 400.0, 256], [0, 0, 1.0]], device=DEVICE).repeat(1, images, 1, 1)
+    values["backgrounds"] = torch.zeros(1, images, 3, device=DEVICE)
+    args = list(compositor_inputs(renderer(False), values, dict(width=size, height=size)))
+    args[2] = torch.full_like(args[2], 4.0)  # alpha = 0.99 at every pixel
+    _, points, ranges, state, contributors, replay = _native.rasterize_forward(*args, replay=True)
+    assert bool((contributors == 1).all())
+    g = torch.Generator(device=DEVICE).manual_seed(3)
+    normals = torch.rand(images, size, size, 3, generator=g, device=DEVICE) + 0.5
+    saved = (*args[:4], args[6], points, ranges, state, contributors)
+    geometry = _native.rasterize_backward(*saved, [None, None, None, normals, None], size, size,
+                                          False, *args[10:12], replay=replay)[0]
+    expected = float(torch.tensor(0.99)) * normals.double().sum((1, 2))
+    error = (geometry[:, 11:14].double() - expected) / expected
+    rms = float(error.square().mean().sqrt())
+    print(f"relative error {rms:.2e}", flush=True)
+    assert math.isfinite(rms) and rms <= 6.6e-7
 
 
 def test_a_non_finite_pixel_reaches_only_the_records_it_took():
