@@ -161,6 +161,16 @@ __device__ constexpr float kDirX[4] = {1.0f, 0.70710677f, -4.371139e-08f, -0.707
 __device__ constexpr float kDirY[4] = {0.0f, 0.70710677f, 1.0f, 0.70710677f};
 
 __device__ __forceinline__ float rcp(float x) { return __builtin_amdgcn_rcpf(x); }
+// 1 / (1 - alpha), the factor by which a backward walk's transmittance grows at
+// every record: v_rcp's error of one ulp would add up over the list, so a Newton
+// step refines it (two multiply-adds, exact at alpha = 0). Colours and normals of
+// lists of 130 records are within 1.7e-7 instead of 2.5e-7 of 64 bits on average,
+// those of a tile walked whole as close as those of one replayed in segments; the
+// kernels take 0.5% longer.
+__device__ __forceinline__ float inverse_keep(float alpha) {
+  const float keep = 1.f - alpha, about = rcp(keep);
+  return fmaf(about, fmaf(-keep, about, 1.f), about);
+}
 __device__ __forceinline__ float sin_rev(float t) { return __builtin_amdgcn_sinf(t); }
 __device__ __forceinline__ float cos_rev(float t) { return __builtin_amdgcn_cosf(t); }
 __device__ __forceinline__ float fract(float t) { return __builtin_amdgcn_fractf(t); }
@@ -2033,7 +2043,7 @@ __global__ __launch_bounds__(kTilePixels, (backward_occupancy<Neural, Replay>())
         float grad[NP];  // geometry NG | appearance A | opacity
         float* gg = grad;
         float* ga = grad + NG;
-        const float inv_keep = rcp(1.f - alpha);
+        const float inv_keep = inverse_keep(alpha);
         T *= inv_keep;  // alpha = 0, inv_keep = 1 where the lane does not take the sample
         const float w = T * alpha;
         Shade a;
@@ -2491,7 +2501,7 @@ __device__ __forceinline__ bool replay_step(const Record& rec, const float* p,
   const float s[2] = {v.s[0], v.s[1]};
   // Transmittance in front of the record: alpha = 0, inv_keep = 1 where the
   // lane does not take it.
-  const float inv_keep = rcp(1.f - alpha);
+  const float inv_keep = inverse_keep(alpha);
   const float T = state.x * row_scan_product(inv_keep);
   const float w = T * alpha;
   // dL/dw without the colour, and dL/dz / w (see the depth factors in
