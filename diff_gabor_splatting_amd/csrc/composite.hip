@@ -2240,7 +2240,8 @@ __global__ __launch_bounds__(kTilePixels, (backward_occupancy<Neural, Replay>())
 #endif
 }
 
-// The classic replay backward: the lanes of a wave are 16 records x 4 pixels.
+// The classic replay backward: the lanes of a wave are 16 records x 4 pixels, or
+// of few records 4 x 16.
 //
 // One wave takes one 8x8 quadrant of a tile and walks the quadrant's replay
 // entries (the records that some pixel of it took) from the last to the
@@ -2270,16 +2271,24 @@ __global__ __launch_bounds__(kTilePixels, (backward_occupancy<Neural, Replay>())
 // It is bound by VALU issue: about 170 instructions per step of 64 samples and
 // 150 per chunk around the steps, against 253 per record and wave with a pixel
 // per lane. Measured, kernel alone: 1M surfels at 1920x1080, all maps, 1.145 ->
-// 0.935 ms; 100k at 1024x768, rgb, alpha and depth, 0.446 -> 0.330 ms; 32 views
-// at 512x512 4.63 -> 3.73 ms. The neural adjoint has 54 sums and 55 record
+// 0.887 ms; 100k at 1024x768, rgb, alpha and depth, 0.443 -> 0.302 ms; 32 views
+// at 512x512 4.63 -> 3.57 ms. The neural adjoint has 54 sums and 55 record
 // constants, which leave two waves per SIMD, and stays with a pixel per lane
 // (0.684 ms against 0.714 on 100k surfels at 800x800). An f32 MFMA per four
 // pixels in place of the products with per-pixel values (20 multiply-adds for 6
 // MFMAs) is slower (1.23 ms): each takes its 32 cycles of the SIMD.
 namespace by_record {
 
-constexpr int kChunk = 16;       // records per chunk: one DPP row
-constexpr int kGroups = 64 / 4;  // pixel steps per chunk
+// Records per chunk: a DPP row of 16 lanes, or a quad of four while at most
+// kFewRecords of the quadrant are left. A chunk takes a step of 64 samples for
+// each record that it may hold, so a few records would cost as much as 16; with
+// quads 10k surfels at 1920x1080 (lists of 4 on average) 194 -> 134 us, 100k small
+// ones (11) 203 -> 153 (a pixel per lane 156 and 179), 1M (128) 931 -> 887. Three
+// quads cost about what a chunk of 16 does: at most 4, 8 or 12 in quads 273, 266
+// and 264 us on lists of 23.
+constexpr int kChunk = 16;
+constexpr int kQuad = 4;
+constexpr int kFewRecords = 12;
 
 // A pixel's constants in LDS: position, last contributor (int bits), the
 // term of dL/dalpha that all records share, map gradients (rgb, depth,
@@ -2350,6 +2359,38 @@ __device__ __forceinline__ float row_before(float scan, float base) {
   return r;
 }
 
+// The same over the W lanes of a chunk, of which this one is `slot`. In a quad
+// the lanes whose source lies before it keep their value by a select.
+template <int Control>
+__device__ __forceinline__ float dpp(float v) {
+  return __int_as_float(
+      __builtin_amdgcn_update_dpp(0, __float_as_int(v), Control, 0xf, 0xf, true));
+}
+constexpr int kQuadBefore = 0x90;   // quad_perm:[0,0,1,2]
+constexpr int kQuadTwoBefore = 0x44;  // quad_perm:[0,1,0,1]
+template <int W>
+__device__ __forceinline__ float chunk_product(float v, int slot) {
+  if constexpr (W == kChunk) return row_scan_product(v);
+  const float one = dpp<kQuadBefore>(v);
+  v *= slot >= 1 ? one : 1.f;
+  const float two = dpp<kQuadTwoBefore>(v);
+  return v * (slot >= 2 ? two : 1.f);
+}
+template <int W>
+__device__ __forceinline__ float chunk_sum(float v, int slot) {
+  if constexpr (W == kChunk) return row_scan_sum(v);
+  const float one = dpp<kQuadBefore>(v);
+  v += slot >= 1 ? one : 0.f;
+  const float two = dpp<kQuadTwoBefore>(v);
+  return v + (slot >= 2 ? two : 0.f);
+}
+template <int W>
+__device__ __forceinline__ float chunk_before(float scan, float base, int slot) {
+  if constexpr (W == kChunk) return row_before(scan, base);
+  const float one = dpp<kQuadBefore>(scan);
+  return base + (slot >= 1 ? one : 0.f);
+}
+
 // Sums over the four DPP rows of a wave (lanes l, l ^ 16, l ^ 32, l ^ 48):
 // row r = lane >> 4 ends with values first(r) + j, j < ROW, of its 16
 // records, first(r) = (r >> 1) HALF + (r & 1) ROW.
@@ -2382,14 +2423,14 @@ __device__ __forceinline__ void wave_lds_fence() {
   __builtin_amdgcn_wave_barrier();
 }
 
-// to[j] += v[j] in LDS for j < count, atomically against the workgroup's other
+// to[Stride j] += v[j] in LDS for j < count, atomically against the workgroup's other
 // waves, with integer exchanges: a float LDS atomic takes about 1.5 cycles per
 // lane, which made the whole kernel 30% slower (1M surfels at 1920x1080 1.32
 // against 0.96 ms). A cell's content is taken (0 left in it), added to and put
 // back; if another wave put its sum in between, that sum comes back and is added
 // again. Each time some wave finds nothing to take back, so of the four that may
 // meet at a cell one at least is done with every turn.
-template <int N>
+template <int Stride, int N>
 __device__ __forceinline__ void shared_add(float* to, float (&v)[N], int count) {
   auto exchange = [](float* cell, float value) {
     return __uint_as_float(__hip_atomic_exchange(reinterpret_cast<uint32_t*>(cell),
@@ -2398,11 +2439,11 @@ __device__ __forceinline__ void shared_add(float* to, float (&v)[N], int count) 
   };
 #pragma unroll
   for (int j = 0; j < N; ++j)
-    if (j < count) v[j] += exchange(to + j, 0.f);
+    if (j < count) v[j] += exchange(to + Stride * j, 0.f);
   uint32_t back = 0;
 #pragma unroll
   for (int j = 0; j < N; ++j) {
-    v[j] = j < count ? exchange(to + j, v[j]) : 0.f;
+    v[j] = j < count ? exchange(to + Stride * j, v[j]) : 0.f;
     back |= __float_as_uint(v[j]);
   }
   while (back) {
@@ -2410,8 +2451,8 @@ __device__ __forceinline__ void shared_add(float* to, float (&v)[N], int count) 
 #pragma unroll
     for (int j = 0; j < N; ++j)
       if (__float_as_uint(v[j]) != 0u) {
-        v[j] += exchange(to + j, 0.f);
-        v[j] = exchange(to + j, v[j]);
+        v[j] += exchange(to + Stride * j, 0.f);
+        v[j] = exchange(to + Stride * j, v[j]);
         back |= __float_as_uint(v[j]);
       }
   }
@@ -2485,8 +2526,8 @@ __device__ __forceinline__ void load_record(Record& rec, float* colour_sums, boo
 // took the record. Lanes that do not take it leave their exact zeros through
 // the stand-ins of sample_surface (see there); Masked also zeroes the
 // gradients of such lanes, for quadrants with a non-finite gradient or state.
-template <int Maps, bool Masked>
-__device__ __forceinline__ bool replay_step(const Record& rec, const float* p,
+template <int Maps, bool Masked, int W>
+__device__ __forceinline__ bool replay_step(const Record& rec, int slot, const float* p,
                                             float2& state, float near_plane, float mscale,
                                             float mnear, float* sum) {
   using P = ReplayPixel;
@@ -2502,7 +2543,7 @@ __device__ __forceinline__ bool replay_step(const Record& rec, const float* p,
   // Transmittance in front of the record: alpha = 0, inv_keep = 1 where the
   // lane does not take it.
   const float inv_keep = inverse_keep(alpha);
-  const float T = state.x * row_scan_product(inv_keep);
+  const float T = state.x * chunk_product<W>(inv_keep, slot);
   const float w = T * alpha;
   // dL/dw without the colour, and dL/dz / w (see the depth factors in
   // renderBackward).
@@ -2561,8 +2602,8 @@ __device__ __forceinline__ bool replay_step(const Record& rec, const float* p,
   gs[0] = gq[0] * rec.ap0 + gq[1] * rec.ap1 + gq[2] * rec.ap2 + gq[3] * rec.ap3;
   gs[1] = gq[1] * rec.ap1 + gq[2] * rec.bp2 - gq[3] * rec.ap3;
   // Running sum behind the record, and the state in front of the chunk.
-  const float scan = row_scan_sum(w * gw);
-  const float galpha = mask(T * gw + (p[P::FINAL] - row_before(scan, state.y)) * inv_keep);
+  const float scan = chunk_sum<W>(w * gw, slot);
+  const float galpha = mask(T * gw + (p[P::FINAL] - chunk_before<W>(scan, state.y, slot)) * inv_keep);
   state.x = T;
   state.y += scan;
   if constexpr (Maps == kAllMaps) {
@@ -2710,7 +2751,7 @@ struct Window {
 // The replay walk's backward compositor: one workgroup per tile, or per
 // segment of a split tile (`segments`), one wave per quadrant.
 template <int Maps>
-__global__ __launch_bounds__(kTilePixels, 3) void renderBackward(
+__global__ __launch_bounds__(kTilePixels, Maps == kAllMaps ? 3 : 4) void renderBackward(
     int width, int height, int tw, int th, const float* __restrict__ geometry,
     const float* __restrict__ appearance, const float* __restrict__ opacities,
     const int64_t* __restrict__ primitive_ids, const float* __restrict__ backgrounds,
@@ -2726,7 +2767,7 @@ __global__ __launch_bounds__(kTilePixels, 3) void renderBackward(
   __shared__ __align__(16) Wave<Maps> waves[kTilePixels / 64];
   __shared__ Window<Maps> window;
   __shared__ float2 aside[64];  // where lanes without a pixel state to keep write theirs
-  __shared__ float bg_acc[3];
+  __shared__ float background_sums[kTilePixels / 64][3];
   const int lane = lane_id();
   // (tile, segment) of this workgroup; past the segment count: nothing.
   const int2 piece = segments ? segments[blockIdx.x] : make_int2(order[blockIdx.x], 0);
@@ -2742,7 +2783,31 @@ __global__ __launch_bounds__(kTilePixels, 3) void renderBackward(
   if (threadIdx.x < 5) diag_packing[threadIdx.x] = 0u;
   PackingCounts packing;
 #endif
-  if (threadIdx.x < 3) bg_acc[threadIdx.x] = 0.f;
+  // The replay entries [block_first, block_last) of the tile: all of them, or
+  // one segment's of a split tile.
+  const int2 range = ranges[tile];
+  const int base = seg.length > 0 ? seg.index[tile] : -1;
+  int block_first = 0, block_last = replay_counts[tile];
+  if (base >= 0) {
+    const int* n = seg.index + seg.tiles + base;
+    block_first = piece.y ? n[piece.y - 1] : 0;
+    block_last = n[piece.y];
+  }
+  // They are taken in equal windows, from the last to the first: entries
+  // [last - n, last) of the block.
+  const int total = block_last - block_first;
+  const int windows = (total + kWindow<Maps> - 1) / kWindow<Maps>;
+  const int size = windows ? (total + windows - 1) / windows : 0;
+  auto load_window = [&](int last, int n) {
+    if (int(threadIdx.x) < n) {
+      const int2 e = replay[range.x + block_first + last - n + int(threadIdx.x)];
+      window.ids[threadIdx.x] = e.x;
+      window.words[threadIdx.x] = e.y;
+      window.prims[threadIdx.x] = uint32_t(primitive_ids[e.x]);
+    }
+    for (int i = threadIdx.x; i < n * kSumPitch; i += kTilePixels) window.sums[i] = 0.f;
+  };
+  load_window(total, size);
   // Per pixel (one per lane): its gradients and final state, staged for the
   // steps.
   const TilePixel tp = tile_pixel(tile, width, height, tw, th);
@@ -2762,20 +2827,12 @@ __global__ __launch_bounds__(kTilePixels, 3) void renderBackward(
   for (int c = 0; c < 3; ++c) background_dot += go[c] * backgrounds[tp.image * 3 + c];
   // dL/dalpha_i picks up final_t (go_alpha - background . go_rgb) / (1 - alpha_i).
   const float final_term = final_t * (go[3] - background_dot);
-  // The replay entries [block_first, block_last) of the tile: all of them, or
-  // one segment's of a split tile, which starts from checkpoint c_{k+1}: its
-  // transmittance, and the suffix sum_{later records} w dL/dw from
-  // c_K - c_{k+1} (the map gradients weigh the prefix-sum differences;
-  // distortion through the final m1, m2).
-  const int2 range = ranges[tile];
-  int block_first = 0, block_last = replay_counts[tile];
+  // A segment starts from checkpoint c_{k+1}: its transmittance, and the suffix
+  // sum_{later records} w dL/dw from c_K - c_{k+1} (the map gradients weigh the
+  // prefix-sum differences; distortion through the final m1, m2).
   float suffix = 0.f;
-  if (seg.length > 0 && seg.index[tile] >= 0) {
-    const int base = seg.index[tile];
+  if (base >= 0) {
     const int pieces = segment_count(range.y - range.x, seg.length);
-    const int* n = seg.index + seg.tiles + base;
-    block_first = piece.y ? n[piece.y - 1] : 0;
-    block_last = n[piece.y];
     if (piece.y < pieces - 1 && tp.inside) {
       constexpr int kSlot = kCheckpointFloats * kTilePixels;
       const float* c = seg.state + int64_t(base + piece.y) * kSlot + threadIdx.x;
@@ -2815,20 +2872,22 @@ __global__ __launch_bounds__(kTilePixels, 3) void renderBackward(
     p[3] = make_float4(c8, d8, 2.f * a8 * mnear, c8 * mnear);
     lds.state[lane] = make_float2(T, suffix);
   }
-  __syncthreads();
   // Background gradient: sum over the tile of final T * dL/drgb (once per
   // tile: by its first segment).
   if (piece.y == 0) {
     const float gb[3] = {final_t * go[0], final_t * go[1], final_t * go[2]};
-    const float total = wave_reduce_quads<3>(gb, lane);
+    const float sum = wave_reduce_quads<3>(gb, lane);
     const int param = rs_quad_param<3>(lane);
-    if (param < 3 && total != 0.f) atomicAdd(&bg_acc[param], total);
+    if (param < 3) background_sums[wave][param] = sum;
   }
   __syncthreads();
-  if (threadIdx.x < 3 && bg_acc[threadIdx.x] != 0.f)
-    atomicAdd(grad_backgrounds + tp.image * 3 + threadIdx.x, bg_acc[threadIdx.x]);
+  if (piece.y == 0 && threadIdx.x < 3) {
+    float sum = 0.f;
+#pragma unroll
+    for (int w = 0; w < kTilePixels / 64; ++w) sum += background_sums[w][threadIdx.x];
+    if (sum != 0.f) atomicAdd(grad_backgrounds + tp.image * 3 + threadIdx.x, sum);
+  }
 
-  const int slot = lane & (kChunk - 1), row = lane >> 4;
   auto uniform = [](float v) {
     return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
   };
@@ -2836,8 +2895,6 @@ __global__ __launch_bounds__(kTilePixels, 3) void renderBackward(
   const float centre_x = uniform(float(tp.px - (lane & 7) - 8 * (wave & 1)) + 7.5f);
   const float centre_y = uniform(float(tp.py - (lane >> 3) - 8 * (wave >> 1)) + 7.5f);
   const int quadrant = kReplayPositionBits + wave;
-  // Lane 15 of a row keeps its pixel's state, the others write theirs aside.
-  float2* const state_row = (slot == kChunk - 1 ? lds.state : aside) + row;
 
   // The wave's part of a window of n entries: those its quadrant took.
   auto walk_window = [&](auto masked, int n) {
@@ -2853,16 +2910,24 @@ __global__ __launch_bounds__(kTilePixels, 3) void renderBackward(
       count += __popcll(kept);
     }
     wave_lds_fence();
-    for (int done = 0; done < count; done += kChunk) {
-      const int in_chunk = min(kChunk, count - done);
+    int done = 0;
+    auto chunk = [&](auto width) {
+      constexpr int W = decltype(width)::value;
+      constexpr int kPixels = 64 / W;  // per step
+      const int slot = lane & (W - 1), row = lane / W;
+      const int in_chunk = min(W, count - done);
       const int entry = lds.taken[done + min(slot, in_chunk - 1)];
       const int id = window.ids[entry];
       const uint32_t prim = window.prims[entry];
       const int position = (window.words[entry] & kReplayPositionMask) + 1;
+      done += W;
       Record rec;
       float colour_sums[3];
       load_record(rec, colour_sums, slot < in_chunk, id, prim, position, centre_x, centre_y,
                   geometry, appearance, opacities);
+      // The chunk's last lane keeps its pixel's state, the others write theirs
+      // aside.
+      float2* const states = (slot == W - 1 ? lds.state : aside) + row;
       float sum[S::COUNT];
 #pragma unroll
       for (int i = 0; i < S::COUNT; ++i) sum[i] = 0.f;
@@ -2870,8 +2935,8 @@ __global__ __launch_bounds__(kTilePixels, 3) void renderBackward(
       uint64_t took = 0;
 #endif
 #pragma unroll 1
-      for (int g = 0; g < kGroups; ++g) {
-        const int q = 4 * g + row;
+      for (int g = 0; g < W; ++g) {
+        const int q = kPixels * g + row;
         float p[P::FLOATS];
         const float4* from = reinterpret_cast<const float4*>(lds.pixels + q * P::FLOATS);
 #pragma unroll
@@ -2883,16 +2948,17 @@ __global__ __launch_bounds__(kTilePixels, 3) void renderBackward(
           p[4 * i + 3] = t.w;
         }
         float2 st = lds.state[q];
-        const bool active = replay_step<Maps, kMasked>(rec, p, st, near_plane, mscale, mnear, sum);
+        const bool active =
+            replay_step<Maps, kMasked, W>(rec, slot, p, st, near_plane, mscale, mnear, sum);
         (void)active;
 #ifdef GS_DIAGNOSTICS
         if (active) took |= uint64_t(1) << q;
 #endif
-        state_row[4 * g] = st;
+        states[kPixels * g] = st;
       }
 #ifdef GS_DIAGNOSTICS
-      took |= __shfl_xor(took, 16, 64);
-      took |= __shfl_xor(took, 32, 64);
+#pragma unroll
+      for (int bit = W; bit < 64; bit *= 2) took |= __shfl_xor(took, bit, 64);
       for (int j = 0; j < in_chunk; ++j) {
         const uint64_t taking = __shfl(took, j, 64);
         if (lane == 0 && taking) atomicAdd(&diag_lanes[__popcll(taking)], 1u);
@@ -2901,29 +2967,47 @@ __global__ __launch_bounds__(kTilePixels, 3) void renderBackward(
       packing.flush(diag_packing);
 #endif
       wave_lds_fence();
-      // The record's sums over the four pixel rows, into the tile's.
+      // The record's sums over the pixel rows, into the tile's.
       using R = RowSums<S::COUNT>;
       float part[R::ROW];
       R::reduce(sum, part, lane);
-      float* to = window.sums + entry * kSumPitch + R::first(row);
-      if (slot < in_chunk) shared_add(to, part, R::count(row));
+      const int dpp_row = lane >> 4;
+      float* const to = window.sums + entry * kSumPitch + R::first(dpp_row);
+      const int values = slot < in_chunk ? R::count(dpp_row) : 0;
+      if constexpr (W == kChunk) {
+        if (values) shared_add<1>(to, part, values);
+      } else {
+        // And over the row's four quads: quad b ends with every fourth value
+        // from the b-th.
+        constexpr int kEach = (R::ROW + 3) / 4;
+        const int b = (lane >> 2) & 3;
+        float own[kEach];
+#pragma unroll
+        for (int j = 0; j < kEach; ++j) {
+          own[j] = 0.f;
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            if (4 * j + k >= R::ROW) break;
+            float v = part[4 * j + k];
+            v += dpp<0x128>(v);  // row_ror:8
+            v += dpp<0x124>(v);  // row_ror:4
+            own[j] = b == k ? v : own[j];
+          }
+        }
+        const int count_b = (values - b + 3) / 4;
+        if (count_b > 0) shared_add<4>(to + b, own, count_b);
+      }
+    };
+    while (done < count) {
+      if (count - done > kFewRecords)
+        chunk(std::integral_constant<int, kChunk>{});
+      else
+        chunk(std::integral_constant<int, kQuad>{});
     }
   };
 
-  // Equal windows, from the last to the first.
-  const int total = block_last - block_first;
-  const int windows = (total + kWindow<Maps> - 1) / kWindow<Maps>;
-  const int size = windows ? (total + windows - 1) / windows : 0;
-  for (int last = total; last > 0; last -= size) {
+  for (int last = total; last > 0;) {
     const int n = min(size, last);
-    if (int(threadIdx.x) < n) {
-      const int2 e = replay[range.x + block_first + last - n + int(threadIdx.x)];
-      window.ids[threadIdx.x] = e.x;
-      window.words[threadIdx.x] = e.y;
-      window.prims[threadIdx.x] = uint32_t(primitive_ids[e.x]);
-    }
-    for (int i = threadIdx.x; i < n * kSumPitch; i += kTilePixels) window.sums[i] = 0.f;
-    __syncthreads();
     if (finite_pixels)
       walk_window(std::false_type{}, n);
     else
@@ -2956,7 +3040,11 @@ __global__ __launch_bounds__(kTilePixels, 3) void renderBackward(
       const float v = window.sums[threadIdx.x * kSumPitch + 32];
       if (v != 0.f) global_add(address(grad_opacities + window.prims[threadIdx.x]), v);
     }
-    __syncthreads();  // before the next window overwrites this one
+    last -= size;
+    if (last <= 0) break;
+    __syncthreads();  // every wave is done with this window
+    load_window(last, min(size, last));
+    __syncthreads();
   }
 #ifdef GS_DIAGNOSTICS
   __syncthreads();
