@@ -832,11 +832,12 @@ __device__ __forceinline__ int append_replay(const uint64_t* wave_taken, const i
 
 // Split tiles. A tile whose point list is longer than `length` records (a
 // multiple of kBatch) is replayed by the backward in segments, one
-// workgroup each, unless the image's tiles are walked whole (whole_pays): segment k takes the replay entries the forward appended
-// while walking list records [k length, (k + 1) length). For it the forward
-// writes checkpoints c_1 .. c_K (K = ceil(list length / length)): c_j is the
-// per-pixel prefix state after the first j length records (c_K: the final
-// state before the background), with the replay-list length at that point.
+// workgroup each, unless the image's tiles are walked whole (whole_pays):
+// segment k takes the replay entries the forward appended while walking list
+// records [k length, (k + 1) length). For it the forward writes checkpoints
+// c_1 .. c_K (K = ceil(list length / length)): c_j is the per-pixel prefix state
+// after the first j length records (c_K: the final state before the background),
+// with the replay-list length at that point.
 // The backward of segment k starts from c_{k+1}: its transmittance, and the
 // sum over the later records of w dL/dw, which is linear in the prefix sums,
 // from c_K - c_{k+1} (the backward's running suffix at that point).
@@ -977,64 +978,87 @@ __device__ __forceinline__ int block_inclusive_sum(int v, int* wave_totals, int*
   return before + incl;
 }
 
-// Whether a split render's long tiles are walked whole after all, from the
-// longest list and the number of segments. Up to kSplitAllTiles tiles (about
-// one workgroup per CU) they are split: the segments run on CUs that would
-// idle. Beyond, the segments compete for CUs that are busy anyway, walk records
-// behind the pixels' stops and pay a merge that grows with their number, while
-// splitting saves the walk of the longest list. One long list among short ones
-// decides the length of the whole launch, so all tiles are split or none. The
-// lines are the ratios of both at which the times of 45 scenes of 256 to 2,016
-// tiles part, forward and backward together, split against whole: 640x480 of
-// 30k surfels (longest 227, 3,773 segments) 300 against 241 us, four 256x256
-// views of 10k (372, 3,095) 270 and 226, longest 967 of 7,142 segments 530 and
-// 303, but 1,080 of 3,245 384 and 454, 588 of 1,631 242 and 292. Neural: 328 of
-// 3,468 372 and 320, 1,176 of 11,730 1,227 and 656, but 370 of 3,106 383 and
-// 417, 783 of 3,983 536 and 678. The rule reads the lists on the device, so a
+// Whether an image's long tiles are walked whole after all, from its longest
+// list and its number of segments times the call's images (what the launch
+// would hold if all were alike). Up to kSplitAllTiles tiles (about one workgroup
+// per CU) they are split: the segments run on CUs that would idle. Beyond, the
+// segments compete for CUs that are busy anyway, walk records behind the pixels'
+// stops and pay a merge that grows with their number, while splitting saves the
+// walk of the longest list. One long list among short ones decides the length of
+// the whole launch, so all tiles of an image are split or none. Split and whole
+// round differently, so the images of a call decide for themselves: what one
+// shows changes no bit of another. The rule reads the lists on the device, so a
 // fixed-capacity render decides as the synchronised one does.
+// The lines keep to the side on which splitting never pays. Of 59 drawn scenes of
+// 257 to 2,047 tiles, forward and backward together, split against whole: the 30
+// walked whole 1.3 to 3.7 times as long split (classic, longest 1,085 of 5,703
+// segments, 501 us split and 359 whole; 2,047 of 17,588 1,084 and 291), the 21
+// split 0.8 to 3.2 times (335 of 1,131 238 and 277; 836 of 1,907 374 and 398; but
+// 1,908 of 8,279 636 and 289. Neural: 828 of 3,426 582 and 710, but 1,218 of 8,231
+// 1,018 and 319). What decides there is where the pixels of the longest list stop,
+// which the list's length does not show.
 constexpr int kSplitAllTiles = 256;
 
-__device__ __forceinline__ bool whole_pays(bool neural, int longest, int segments) {
-  return longest <= (neural ? segments / 7 - 100 : max(segments / 5, 170));
+__device__ __forceinline__ bool whole_pays(bool neural, int longest, int64_t segments) {
+  return longest <= (neural ? segments / 7 - 100 : max(segments / 5, int64_t(170)));
 }
 
 // cost: per-tile cost, or null to use the tile's list length from ranges.
 // With seg.length > 0 (the forward of split tiles) it writes the (tile,
 // segment) work list in place of `order`, and assigns each tile longer than
-// seg.length, unless whole_pays, its ceil(length / seg.length) checkpoint
-// slots, in tile order, into seg.index[0 .. tiles) (-1: not split, or past
-// the capacity, which the host sizes so that it is never reached).
+// seg.length, unless whole_pays for its image, its ceil(length / seg.length)
+// checkpoint slots, in tile order, into seg.index[0 .. tiles) (-1: not split, or
+// past the capacity, which the host sizes so that it is never reached).
 __global__ __launch_bounds__(kOrderBlock) void tile_order_kernel(const int* __restrict__ cost,
                                                                  const int2* __restrict__ ranges,
-                                                                 int tiles,
+                                                                 int tiles, int images,
                                                                  int* __restrict__ order,
                                                                  bool neural, Segments seg) {
   __shared__ int count[kOrderBuckets];
   __shared__ int next[kOrderBuckets];
   __shared__ int scan[kOrderBlock];
   if (seg.length > 0) {
-    int longest_whole = seg.length;
-    if (tiles > kSplitAllTiles) {
-      int own = 0, longest = 0;
-      for (int t = threadIdx.x; t < tiles; t += kOrderBlock) {
-        const int length = ranges[t].y - ranges[t].x;
-        own += length > seg.length ? segment_count(length, seg.length) : 0;
-        longest = max(longest, length);
+    // The longest list that is walked whole, per image; with more than
+    // kOrderBlock images whole_pays holds for all of them.
+    __shared__ int longest_whole[kOrderBlock];
+    const int per_image = tiles / images;
+    if (tiles > kSplitAllTiles && images <= kOrderBlock) {
+      int* const longest = longest_whole;
+      int* const segments = scan;
+      longest[threadIdx.x] = segments[threadIdx.x] = 0;
+      __syncthreads();
+      for (int first = threadIdx.x & ~63; first < tiles; first += kOrderBlock) {
+        const int t = first + lane_id();
+        const int length = t < tiles ? ranges[t].y - ranges[t].x : 0;
+        const int own = length > seg.length ? segment_count(length, seg.length) : 0;
+        const int image = first / per_image;
+        if (image == min(first + 63, tiles - 1) / per_image) {  // one image's tiles
+          const int most = wave_max(length);
+          const int sum = wave_inclusive_sum(own);
+          if (lane_id() == 63) {
+            atomicMax(&longest[image], most);
+            atomicAdd(&segments[image], sum);
+          }
+        } else if (own) {
+          atomicMax(&longest[t / per_image], length);
+          atomicAdd(&segments[t / per_image], own);
+        }
       }
-      if (threadIdx.x == 0) next[0] = 0;
-      int segments;
-      block_inclusive_sum(own, scan, &segments);
-      longest = wave_max(longest);
-      if (lane_id() == 0) atomicMax(&next[0], longest);
       __syncthreads();
-      if (whole_pays(neural, next[0], segments)) longest_whole = INT_MAX;
-      __syncthreads();
+      const bool whole = whole_pays(neural, longest[threadIdx.x],
+                                    int64_t(segments[threadIdx.x]) * images);
+      longest[threadIdx.x] = whole ? INT_MAX : seg.length;
+    } else {
+      longest_whole[threadIdx.x] = tiles > kSplitAllTiles ? INT_MAX : seg.length;
     }
+    __syncthreads();
     int carry = 0;
     for (int first = 0; first < tiles; first += kOrderBlock) {
       const int t = first + threadIdx.x;
       const int length = t < tiles ? ranges[t].y - ranges[t].x : 0;
-      const int slots = length > longest_whole ? segment_count(length, seg.length) : 0;
+      const int image = t < tiles ? t / per_image : 0;
+      const int slots = length > longest_whole[min(image, kOrderBlock - 1)]
+                            ? segment_count(length, seg.length) : 0;
       int chunk;
       const int base = carry + block_inclusive_sum(slots, scan, &chunk) - slots;
       if (t < tiles) seg.index[t] = (slots > 0 && base + slots <= seg.capacity) ? base : -1;
@@ -3187,8 +3211,8 @@ int render_forward(int32_t neural, const float* geometry, const float* appearanc
     else run(tile_probe_kernel<false>);
     GS_LAUNCHED("tile_probe_kernel");
   }
-  tile_order_kernel<<<1, kOrderBlock, 0, s>>>(probed ? probe : nullptr, r, tiles, order,
-                                              neural != 0, seg);
+  tile_order_kernel<<<1, kOrderBlock, 0, s>>>(probed ? probe : nullptr, r, tiles, int(images),
+                                              order, neural != 0, seg);
   GS_LAUNCHED("tile_order_kernel");
   int2* lists = reinterpret_cast<int2*>(replay);
   const unsigned blocks = unsigned(seg.length ? tiles + seg.capacity : tiles);
@@ -3401,7 +3425,7 @@ int gs_render_backward(int32_t neural, const float* geometry, const float* appea
       GS_LAUNCHED("tile_last_kernel");
     }
     tile_order_kernel<<<1, kOrderBlock, 0, s>>>(replay ? replay_counts : w.tile_last, r, tiles,
-                                                w.order, neural != 0, seg);
+                                                int(images), w.order, neural != 0, seg);
     GS_LAUNCHED("tile_order_kernel");
   }
   const int2* lists = reinterpret_cast<const int2*>(replay);

@@ -450,9 +450,11 @@ int gs_render_forward(int32_t neural, const float* geometry, const float* appear
  * in the reference, which walks each tile in one thread block. A tile whose
  * point list is longer than segment_length records is split into
  * K = ceil(length / segment_length) segments with K checkpoint slots,
- * assigned in tile order; of more than 256 tiles none is split where the
- * longest list is short against the number of segments, which the forward
- * decides on the device. The forward walks every segment in its own
+ * assigned in tile order; with more than 256 tiles in the call none of an
+ * image is split where its longest list is short against its number of
+ * segments times the call's images, which the forward decides on the device
+ * for each image by itself: what another image shows changes none of its
+ * bits, the number and size of the images may. The forward walks every segment in its own
  * workgroup, with the transmittance in front of it taken as 1, and a
  * second kernel merges the segments per pixel in list order, in closed
  * form, or by walking a segment again with the true transmittance where

@@ -11,7 +11,7 @@ each from a checkpoint the merge wrote.
   longer than the segment length, non-decreasing replay lengths ending at
   the tile's replay count, and a last checkpoint equal to the saved state.
 * Gradients of a scene whose tiles are split match the float64 oracle.
-* Beyond 256 tiles the lists decide whether the long tiles are split.
+* Beyond 256 tiles an image's lists decide whether its long tiles are split.
 """
 
 import pytest
@@ -220,11 +220,17 @@ def test_slots_past_capacity_leave_later_tiles_unsplit(method, monkeypatch):
         assert err <= 1e-3 * scale + 1e-12, f"{name}: max error {err:.3e}, scale {scale:.3e}"
 
 
-def walked_whole(method, tiles, longest, segments):
-    """The compositor's rule (whole_pays in composite.hip)."""
-    if tiles <= 256:
-        return False
-    return longest <= (segments // 7 - 100 if method == "neural" else max(segments // 5, 170))
+def walked_whole(method, lengths, images, segment):
+    """The compositor's rule (whole_pays in composite.hip), per image, from the
+    lists' lengths."""
+    if lengths.numel() <= 256:
+        return [False] * images
+    out = []
+    for own in lengths.reshape(images, -1):
+        segments = images * int(((own + segment - 1) // segment)[own > segment].sum())
+        out.append(int(own.max()) <= (segments // 7 - 100 if method == "neural"
+                                      else max(segments // 5, 170)))
+    return out
 
 
 @pytest.mark.parametrize("method", ["classic", "neural"])
@@ -235,8 +241,8 @@ def walked_whole(method, tiles, longest, segments):
     (1, 272, 256, 0.15, False),
 ])
 def test_whole_or_split(method, cameras, width, height, spread, whole, monkeypatch):
-    """Beyond 256 tiles the lists decide on the device whether the long tiles
-    are split, all or none: the decision is the rule's, the same in a
+    """Beyond 256 tiles an image's lists decide on the device whether its long
+    tiles are split, all or none: the decision is the rule's, the same in a
     fixed-capacity render (same bits), and the results are the unsplit
     render's to float32 rounding, as for every split."""
     raw = random_scene(method, scenes=1, cameras=cameras, n=1500, width=width, height=height,
@@ -251,9 +257,7 @@ def test_whole_or_split(method, cameras, width, height, spread, whole, monkeypat
     _, _, ranges, _, contributors, (_, _, (length, _, index)) = seen[-1]
     tiles = ranges.shape[0]
     lengths = (ranges[:, 1] - ranges[:, 0]).long()
-    segments = int(((lengths + length - 1) // length)[lengths > length].sum())
-    print(f"longest {int(lengths.max())}, {segments} segments of {tiles} tiles", flush=True)
-    assert walked_whole(method, tiles, int(lengths.max()), segments) == whole
+    assert walked_whole(method, lengths, cameras, length) == [whole] * cameras
     assert torch.equal(index[:tiles] >= 0, (lengths > length) & (not whole))
     capacity = int(lengths.sum()) + 777
     with torch.no_grad(), fixed_capacity(capacity):
@@ -268,6 +272,38 @@ def test_whole_or_split(method, cameras, width, height, spread, whole, monkeypat
         scale = float(b.abs().max())
         err = float((a - b).abs().max())
         assert err <= 1e-3 * scale + 1e-12, f"{name}: max error {err:.3e}, scale {scale:.3e}"
+
+
+@pytest.mark.parametrize("method", ["classic", "neural"])
+def test_images_decide_for_themselves(method, monkeypatch):
+    """The other images' lists change no bit of an image, however they fall out
+    themselves: taken over all images, the lists would decide differently for
+    even scenes and for three whose surfels crowd in the middle."""
+    width, height, images = 250, 255, 4
+    raw = random_scene(method, scenes=images, cameras=1, n=1500, width=width, height=height,
+                       seed=3, focal=330.0)
+    seen = spy_forward(monkeypatch)
+    first, decisions, together = [], [], []
+    for spread in (1.0, 0.15):
+        values = {k: v.clone().to(DEVICE) for k, v in raw.items()}
+        values["means"][1:, :, :2] *= spread
+        values["means"].requires_grad_()  # the segments are returned for a backward
+        maps = maps_from_result(renderer(method)(**values, width=width, height=height)).detach()
+        _, _, ranges, state, contributors, (_, _, (length, _, index)) = seen[-1]
+        lengths = (ranges[:, 1] - ranges[:, 0]).long()
+        whole = walked_whole(method, lengths, images, length)
+        split = (index[:len(lengths)] >= 0).reshape(images, -1)
+        for image in range(images):
+            own = lengths.reshape(images, -1)[image] > length
+            assert torch.equal(split[image], own & (not whole[image]))
+        first.append((maps[0], state[0], contributors[0], split[0]))
+        decisions.append(whole)
+        together.append(walked_whole(method, lengths, 1, length))
+        print(f"spread {spread}: {whole}, together {together[-1]}", flush=True)
+    assert together == [[True], [False]]
+    assert decisions == [[True] * 4, [True, False, False, False]]
+    for a, b in zip(*first):
+        assert torch.equal(a, b)
 
 
 @pytest.mark.parametrize("length", [64, 192])
