@@ -979,8 +979,8 @@ __device__ __forceinline__ int block_inclusive_sum(int v, int* wave_totals, int*
 }
 
 // Whether an image's long tiles are walked whole after all, from its longest
-// list and its number of segments times the call's images (what the launch
-// would hold if all were alike). Up to kSplitAllTiles tiles (about one workgroup
+// list and the kBatch-record segments of its long lists, whatever the segments'
+// length, times the call's images (what the launch would hold if all were alike). Up to kSplitAllTiles tiles (about one workgroup
 // per CU) they are split: the segments run on CUs that would idle. Beyond, the
 // segments compete for CUs that are busy anyway, walk records behind the pixels'
 // stops and pay a merge that grows with their number, while splitting saves the
@@ -996,7 +996,10 @@ __device__ __forceinline__ int block_inclusive_sum(int v, int* wave_totals, int*
 // split 0.8 to 3.2 times (335 of 1,131 238 and 277; 836 of 1,907 374 and 398; but
 // 1,908 of 8,279 636 and 289. Neural: 828 of 3,426 582 and 710, but 1,218 of 8,231
 // 1,018 and 319). What decides there is where the pixels of the longest list stop,
-// which the list's length does not show.
+// which the list's length does not show. Where the images of a call decided
+// differently (eight scenes) it took 0.79 to 1.08 of all split. Counted in segments
+// of 192 records instead, 17 of 30 other scenes would have been split that took 1.2
+// to 4.3 times as long so; of 512, eight of 20 that took 1.0 to 2.2 times.
 constexpr int kSplitAllTiles = 256;
 
 __device__ __forceinline__ bool whole_pays(bool neural, int longest, int64_t segments) {
@@ -1030,7 +1033,7 @@ __global__ __launch_bounds__(kOrderBlock) void tile_order_kernel(const int* __re
       for (int first = threadIdx.x & ~63; first < tiles; first += kOrderBlock) {
         const int t = first + lane_id();
         const int length = t < tiles ? ranges[t].y - ranges[t].x : 0;
-        const int own = length > seg.length ? segment_count(length, seg.length) : 0;
+        const int own = length > kBatch ? segment_count(length, kBatch) : 0;
         const int image = first / per_image;
         if (image == min(first + 63, tiles - 1) / per_image) {  // one image's tiles
           const int most = wave_max(length);

@@ -220,14 +220,14 @@ def test_slots_past_capacity_leave_later_tiles_unsplit(method, monkeypatch):
         assert err <= 1e-3 * scale + 1e-12, f"{name}: max error {err:.3e}, scale {scale:.3e}"
 
 
-def walked_whole(method, lengths, images, segment):
+def walked_whole(method, lengths, images):
     """The compositor's rule (whole_pays in composite.hip), per image, from the
-    lists' lengths."""
+    lists' lengths, in segments of 64 records."""
     if lengths.numel() <= 256:
         return [False] * images
     out = []
     for own in lengths.reshape(images, -1):
-        segments = images * int(((own + segment - 1) // segment)[own > segment].sum())
+        segments = images * int(((own + 63) // 64)[own > 64].sum())
         out.append(int(own.max()) <= (segments // 7 - 100 if method == "neural"
                                       else max(segments // 5, 170)))
     return out
@@ -257,7 +257,7 @@ def test_whole_or_split(method, cameras, width, height, spread, whole, monkeypat
     _, _, ranges, _, contributors, (_, _, (length, _, index)) = seen[-1]
     tiles = ranges.shape[0]
     lengths = (ranges[:, 1] - ranges[:, 0]).long()
-    assert walked_whole(method, lengths, cameras, length) == [whole] * cameras
+    assert walked_whole(method, lengths, cameras) == [whole] * cameras
     assert torch.equal(index[:tiles] >= 0, (lengths > length) & (not whole))
     capacity = int(lengths.sum()) + 777
     with torch.no_grad(), fixed_capacity(capacity):
@@ -291,19 +291,43 @@ def test_images_decide_for_themselves(method, monkeypatch):
         maps = maps_from_result(renderer(method)(**values, width=width, height=height)).detach()
         _, _, ranges, state, contributors, (_, _, (length, _, index)) = seen[-1]
         lengths = (ranges[:, 1] - ranges[:, 0]).long()
-        whole = walked_whole(method, lengths, images, length)
+        whole = walked_whole(method, lengths, images)
         split = (index[:len(lengths)] >= 0).reshape(images, -1)
         for image in range(images):
             own = lengths.reshape(images, -1)[image] > length
             assert torch.equal(split[image], own & (not whole[image]))
         first.append((maps[0], state[0], contributors[0], split[0]))
         decisions.append(whole)
-        together.append(walked_whole(method, lengths, 1, length))
+        together.append(walked_whole(method, lengths, 1))
         print(f"spread {spread}: {whole}, together {together[-1]}", flush=True)
     assert together == [[True], [False]]
     assert decisions == [[True] * 4, [True, False, False, False]]
     for a, b in zip(*first):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("method", ["classic", "neural"])
+@pytest.mark.parametrize("length", [64, 192, 320])
+@pytest.mark.parametrize("spread", [1.0, 0.15])
+def test_decision_does_not_depend_on_the_segment_length(method, length, spread, monkeypatch):
+    """Longer segments are fewer, but the lists that decide are the same: walked
+    whole at one segment length, an image is so at every length."""
+    width, height, images = 250, 255, 5
+    raw = random_scene(method, scenes=1, cameras=images, n=3000, width=width, height=height,
+                       seed=3, focal=330.0)
+    raw["means"][..., :2] *= spread
+    values = {k: v.to(DEVICE) for k, v in raw.items()}
+    values["means"].requires_grad_()  # the segments are returned for a backward
+    monkeypatch.setattr(_native, "SPLIT_LENGTH", length)
+    seen = spy_forward(monkeypatch)
+    renderer(method)(**values, width=width, height=height)
+    _, _, ranges, _, _, (_, _, (used, _, index)) = seen[-1]
+    lengths = (ranges[:, 1] - ranges[:, 0]).long()
+    whole = walked_whole(method, lengths, images)
+    assert used == length and whole == [spread == 1.0] * images
+    print(f"longest {int(lengths.max())}", flush=True)
+    assert int(lengths.max()) > 320
+    assert torch.equal(index[:len(lengths)] >= 0, (lengths > length) & (not whole[0]))
 
 
 @pytest.mark.parametrize("length", [64, 192])
