@@ -49,10 +49,9 @@ int sort_items(int64_t m) {
 }
 constexpr int kDigitBits = 8;
 constexpr int kBins = 1 << kDigitBits;
-// Multi-workgroup passes of 32-bit keys may take digits of up to
-// kWideDigitBits bits (kWideBins bins) when that saves a pass: the 9-bit
-// block-id sort of a 1080p image (510 tile blocks) then takes one pass
-// instead of two. (Digits of 11 bits, which would sort 32-bit depth keys in
+// Sorts of 32-bit keys may take digits of up to kWideDigitBits bits (kWideBins
+// bins) when that saves a pass: the 9-bit block-id sort of a 1080p image (510
+// tile blocks) then takes one pass instead of two. (Digits of 11 bits, which would sort 32-bit depth keys in
 // three passes, measured slower: 2048-bin histograms and scans per span
 // cost more than the pass they save.) The digit-major counts are sized for
 // kWideBins.
@@ -489,8 +488,9 @@ int radix_sort(const Key* keys_in, Key* keys_out, const int* values_in, int* val
     GS_LAUNCHED("copy_pairs_kernel");
     return GS_OK;
   }
-  // Wider digits for 32-bit keys when they save a pass.
-  if (sizeof(Key) == 4) {
+  // Wider digits when they save a pass, and keys alone: of 32-bit keys only.
+  constexpr bool kNarrow = sizeof(Key) == 4;
+  if (kNarrow) {
     const int wide_passes = int(ceil_div(bits_total, kWideDigitBits));
     if (wide_passes < passes) {
       passes = wide_passes;
@@ -505,8 +505,10 @@ int radix_sort(const Key* keys_in, Key* keys_out, const int* values_in, int* val
         kernel<<<1, kLocalBlock, 0, s>>>(keys_in, values_in, keys_out, values_out, m, live,
                                          begin_bit, end_bit, passes, digit_bits);
       };
-      if (values_in) launch(local_sort_kernel<Key, true, I, B>);
-      else launch(local_sort_kernel<Key, false, I, B>);
+      if constexpr (kNarrow) {
+        if (!values_in) return launch(local_sort_kernel<Key, false, I, B>);
+      }
+      launch(local_sort_kernel<Key, true, I, B>);
     };
     auto by_length = [&](auto bins_tag) {
       if (m <= kLocalBlock) local(std::integral_constant<int, 1>{}, bins_tag);
@@ -514,8 +516,12 @@ int radix_sort(const Key* keys_in, Key* keys_out, const int* values_in, int* val
       else if (m <= 4 * kLocalBlock) local(std::integral_constant<int, 4>{}, bins_tag);
       else local(std::integral_constant<int, kLocalItems>{}, bins_tag);
     };
-    if (bins == kBins) by_length(std::integral_constant<int, kBins>{});
-    else by_length(std::integral_constant<int, kWideBins>{});
+    if constexpr (kNarrow) {
+      if (bins == kBins) by_length(std::integral_constant<int, kBins>{});
+      else by_length(std::integral_constant<int, kWideBins>{});
+    } else {
+      by_length(std::integral_constant<int, kBins>{});
+    }
     GS_LAUNCHED("local_sort_kernel");
     return GS_OK;
   }
@@ -535,12 +541,14 @@ int radix_sort(const Key* keys_in, Key* keys_out, const int* values_in, int* val
     };
     auto downsweep = [&](auto items_tag, auto bins_tag) {
       constexpr int I = decltype(items_tag)::value, B = decltype(bins_tag)::value;
-      if (values_in)
-        radix_downsweep_kernel<Key, I, true, B><<<unsigned(spans), kSortBlock, 0, s>>>(
-            src_k, src_v, dst_k, dst_v, m, live, shift, bits, w.counts, w.totals, spans);
-      else
-        radix_downsweep_kernel<Key, I, false, B><<<unsigned(spans), kSortBlock, 0, s>>>(
-            src_k, src_v, dst_k, dst_v, m, live, shift, bits, w.counts, w.totals, spans);
+      auto launch = [&](auto kernel) {
+        kernel<<<unsigned(spans), kSortBlock, 0, s>>>(src_k, src_v, dst_k, dst_v, m, live, shift,
+                                                      bits, w.counts, w.totals, spans);
+      };
+      if constexpr (kNarrow) {
+        if (!values_in) return launch(radix_downsweep_kernel<Key, I, false, B>);
+      }
+      launch(radix_downsweep_kernel<Key, I, true, B>);
     };
     auto run = [&](auto items_tag, auto bins_tag) {
       constexpr int B = decltype(bins_tag)::value;
@@ -559,8 +567,13 @@ int radix_sort(const Key* keys_in, Key* keys_out, const int* values_in, int* val
       if (items == 8) return run(std::integral_constant<int, 8>{}, bins_tag);
       return run(std::integral_constant<int, 16>{}, bins_tag);
     };
-    const int status = bins == kBins ? by_items(std::integral_constant<int, kBins>{})
-                                     : by_items(std::integral_constant<int, kWideBins>{});
+    auto by_bins = [&] {
+      if constexpr (kNarrow) {
+        if (bins != kBins) return by_items(std::integral_constant<int, kWideBins>{});
+      }
+      return by_items(std::integral_constant<int, kBins>{});
+    };
+    const int status = by_bins();
     if (status != GS_OK) return status;
     src_k = dst_k;
     src_v = dst_v;
