@@ -42,7 +42,7 @@ REPLAY_MAX_ENTRIES = 2**28 - 1
 # list, so tiles longer than SPLIT_LENGTH records are composited (and their
 # backward replayed) in segments of that many records, one workgroup each;
 # beyond 256 tiles only where that pays, which the forward decides on the
-# device from the longest list and the number of segments.
+# device, per image, from its longest list and the length of its long lists.
 # The segment length does not depend on the intersection count, and the
 # checkpoint slots are at most SPLIT_MAX_SLOTS, so a render into a
 # fixed-capacity point list splits its tiles exactly as the synchronised

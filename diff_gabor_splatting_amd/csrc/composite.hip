@@ -64,8 +64,9 @@ struct DiagnosticTargets {
   // times 64 lanes; the backward's processed (record, wave) pairs and the
   // wave steps they would take with each 32-lane half (8x4) or each 16-lane
   // block (4x4) of the quadrant walking its own records: at best (per batch,
-  // the largest count of any half or block) and in list order (records
-  // taken by one half or block packed between those taken by several).
+  // by_record per chunk, the largest count of any half or block) and in list
+  // order (records taken by one half or block packed between those taken by
+  // several).
   unsigned long long* counters;
 };
 
@@ -978,17 +979,18 @@ __device__ __forceinline__ int block_inclusive_sum(int v, int* wave_totals, int*
   return before + incl;
 }
 
-// Whether an image's long tiles are walked whole after all, from its longest
-// list and the kBatch-record segments of its long lists, whatever the segments'
-// length, times the call's images (what the launch would hold if all were alike). Up to kSplitAllTiles tiles (about one workgroup
-// per CU) they are split: the segments run on CUs that would idle. Beyond, the
-// segments compete for CUs that are busy anyway, walk records behind the pixels'
-// stops and pay a merge that grows with their number, while splitting saves the
-// walk of the longest list. One long list among short ones decides the length of
-// the whole launch, so all tiles of an image are split or none. Split and whole
-// round differently, so the images of a call decide for themselves: what one
-// shows changes no bit of another. The rule reads the lists on the device, so a
-// fixed-capacity render decides as the synchronised one does.
+// Whether an image's long tiles are walked whole after all, from its longest list
+// and the kBatch-record segments of its long lists, whatever the segments' length,
+// times the call's images (what the launch would hold if all were alike). Up to
+// kSplitAllTiles tiles (about one workgroup per CU) they are split: the segments
+// run on CUs that would idle. Beyond, the segments compete for CUs that are busy
+// anyway, walk records behind the pixels' stops and pay a merge that grows with
+// their number, while splitting saves the walk of the longest list. One long list
+// among short ones decides the length of the whole launch, so all tiles of an
+// image are split or none. Split and whole round differently, so the images of a
+// call decide for themselves: what one shows changes no bit of another. The rule
+// reads the lists on the device, so a fixed-capacity render decides as the
+// synchronised one does.
 // The lines keep to the side on which splitting never pays. Of 59 drawn scenes of
 // 257 to 2,047 tiles, forward and backward together, split against whole: the 30
 // walked whole 1.3 to 3.7 times as long split (classic, longest 1,085 of 5,703
@@ -998,7 +1000,7 @@ __device__ __forceinline__ int block_inclusive_sum(int v, int* wave_totals, int*
 // 1,018 and 319). What decides there is where the pixels of the longest list stop,
 // which the list's length does not show. Where the images of a call decided
 // differently (eight scenes) it took 0.79 to 1.08 of all split. Counted in segments
-// of 192 records instead, 17 of 30 other scenes would have been split that took 1.2
+// of 192 records instead, 17 of 30 other scenes would have been split that took 1.1
 // to 4.3 times as long so; of 512, eight of 20 that took 1.0 to 2.2 times.
 constexpr int kSplitAllTiles = 256;
 

@@ -545,8 +545,9 @@ int gs_render_backward(int32_t neural, const float* geometry, const float* appea
  * lanes; [2] the (record, wave) pairs the backward processed; the wave
  * steps those would take if each 32-lane half (8x4 pixels) or each 16-lane
  * block (4x4) of the wave's quadrant walked its own records: [3] halves and
- * [4] blocks at best (per batch the largest number of records any half or
- * block takes), [5] halves and [6] blocks in list order (records taken by
+ * [4] blocks at best (the largest number of records any half or block takes,
+ * per batch of 64 or, in the classic replay, per chunk of 16 or four),
+ * [5] halves and [6] blocks in list order (records taken by
  * one half or block packed between records taken by several); [7] unused.
  * These cost a few instructions per processed (record, wave), so the
  * diagnostics library is for measurement only.                          */
