@@ -988,9 +988,9 @@ __device__ __forceinline__ int block_inclusive_sum(int v, int* wave_totals, int*
 // their number, while splitting saves the walk of the longest list. One long list
 // among short ones decides the length of the whole launch, so all tiles of an
 // image are split or none. Split and whole round differently, so the images of a
-// call decide for themselves: what one shows changes no bit of another. The rule
-// reads the lists on the device, so a fixed-capacity render decides as the
-// synchronised one does.
+// call decide for themselves: what one shows changes no bit of another while the
+// slots last. The rule reads the lists on the device, so a fixed-capacity render
+// decides as the synchronised one does.
 // The lines keep to the side on which splitting never pays. Of 59 drawn scenes of
 // 257 to 2,047 tiles, forward and backward together, split against whole: the 30
 // walked whole 1.3 to 3.7 times as long split (classic, longest 1,085 of 5,703

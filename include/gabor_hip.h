@@ -453,9 +453,9 @@ int gs_render_forward(int32_t neural, const float* geometry, const float* appear
  * assigned in tile order; with more than 256 tiles in the call none of an
  * image is split where its longest list is short against the records of its
  * long lists times the call's images, which the forward decides on the device
- * for each image by itself, whatever the segment length: what another image
- * shows changes none of its bits, the number and size of the images may. The
- * forward walks every segment in its own
+ * for each image by itself, whatever the segment length: while the slots
+ * last, what another image shows changes none of its bits; the number and size
+ * of the images may. The forward walks every segment in its own
  * workgroup, with the transmittance in front of it taken as 1, and a
  * second kernel merges the segments per pixel in list order, in closed
  * form, or by walking a segment again with the true transmittance where
